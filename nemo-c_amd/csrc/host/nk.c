@@ -9,11 +9,11 @@
 
 static int g_force = 0;
 static int g_split = -1; /* many-row residual updates: -1 K split chosen by tile count, 0 never, 1 always */
-static int g_mx_tile = -1; /* many-row tile: -1 by tile count, else 0 128x128, 1 64x128, 2 64x64 where it divides */
+static int g_mx_tile = -1; /* many-row tile: -1 by estimate, else an index of mx_tile where it applies */
 
 int nk_gemm_mx_tile(int t) {
     const int prev = g_mx_tile;
-    g_mx_tile = t < 0 || t > 2 ? -1 : t;
+    g_mx_tile = t < 0 || t > 5 ? -1 : t;
     return prev;
 }
 
@@ -142,59 +142,84 @@ typedef struct {
     float *fold_out;        /* receives A with the update applied */
 } ln_pro_t;
 
-/* Many-row GEMM on the direct-to-LDS MFMA kernels (kernels/nk_mx.hip).  Tile choice: the largest
- * of 128x128, 64x128, 64x64 whose tile count reaches about 400 workgroups; otherwise the smallest
- * tile that divides the output columns.  Residual updates (accumulate, no bias, no activation, no
- * row map) run on the _acc kernels: their K sum is blocked (mx_kblocks), below ~400 tiles K is
- * split one block per workgroup, and the sums go to partial rows in the scratch (nparts of them,
- * same bits either way); *pend then describes the update still to apply (NkFoldArgs).
- * Returns 1 when no tile divides the output columns (the caller falls back), -2 when a fixed
- * scratch region is too small, else the launch status. */
 typedef struct {
     float *ws; /* fixed region (no allocation; a launch that needs more is refused), or NULL */
     size_t ws_floats;
 } mx_scratch_t;
 
+/* 2^32 / d rounded up (0 for d = 1): the kernels' division of tile numbers below 65536 */
+static uint32_t recip32(uint32_t d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0; }
+
+/* The many-row kernels (kernels/nk_mx.hip).  A launch runs in rounds of `slots` workgroups (256 CUs x
+ * workgroups per CU); a round takes about fix + step x K steps (64 columns) microseconds, fix1 + step1
+ * x K steps when no CU has more than one workgroup.  Index 0: split-row A, fitted to FF up, FF down,
+ * QKV, pw1 and out at 18 to 3584 rows (graph replays, within 15%); 1: f32 A (the split costs vector
+ * work per step), fitted to the subsampling's GEMMs and joint.enc at 64 to 40128 rows. */
+typedef struct {
+    const char *tile;
+    uint16_t bm, bn, slots;
+    struct { float fix, step, fix1, step1; } us[2]; /* fix 0: not built for this form */
+} mx_tile_t;
+static const mx_tile_t mx_tile[] = { /* in the order of nk_gemm_mx_tile's numbers */
+    { "128x256", 128, 256, 256, { { 5.0f, 1.45f, 5.0f, 1.45f }, { 0 } } },
+    { "64x128", 64, 128, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
+    { "64x64", 64, 64, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
+    { "32x64", 32, 64, 256, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
+    { "32x32", 32, 32, 256, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
+    { "64x128d", 64, 128, 256, { { 2.5f, 0.63f, 2.5f, 0.63f }, { 0 } } },
+};
+#define MX_TILES ((int)(sizeof mx_tile / sizeof *mx_tile))
+#define MX_THREADS 512 /* every kernel: 8 computing wavefronts, or 4 that compute and 4 that load */
+
+static uint32_t mx_tiles(const mx_tile_t *t, uint32_t M, uint32_t nout, int glu) {
+    const uint32_t cols = glu ? t->bn / 2u : t->bn;
+    if (nout % cols || (glu && t->bn < 64)) return 0; /* a GLU wavefront holds 16 value and 16 gate columns */
+    return (M + t->bm - 1) / t->bm * (nout / cols);
+}
+
+/* the tile of an (M, nout, K) GEMM, NULL when none divides the output columns; kb: K blocks that may
+ * run as workgroups of their own (residual updates) */
+static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, int glu, uint32_t kb) {
+    const mx_tile_t *best = NULL;
+    float least = 0;
+    if (nout % (glu ? 32 : 64)) return NULL;
+    for (int i = 0; i < MX_TILES; ++i) {
+        const mx_tile_t *t = &mx_tile[i];
+        const uint32_t tiles = t->us[f32].fix > 0 ? mx_tiles(t, M, nout, glu) : 0;
+        if (!tiles) continue;
+        if (i == g_mx_tile) return t;
+        const uint32_t wgs = tiles * kb;
+        const float steps = (float)(K / kb) / NK_MX_KS;
+        const float us = wgs <= 256 ? t->us[f32].fix1 + t->us[f32].step1 * steps
+                                    : (float)((wgs + t->slots - 1) / t->slots) * (t->us[f32].fix + t->us[f32].step * steps);
+        if (!best || us < least) {
+            best = t;
+            least = us;
+        }
+    }
+    return best;
+}
+
+/* Many-row GEMM.  Residual updates (accumulate, no bias, no activation, no row map) run on the _acc
+ * kernels: their K sum is blocked (mx_kblocks), and split-row ones run one K block per workgroup (f32
+ * ones below 400 tiles); the sums go to partial rows in the scratch (nparts of them, same bits either
+ * way); *pend then describes the update still to apply (NkFoldArgs).
+ * Returns 1 when no tile divides the output columns (the caller falls back), -2 when a fixed
+ * scratch region is too small, else the launch status. */
 static int launch_mx_s(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid,
                        const mx_scratch_t *sc, nk_resid_t *pend) {
-    /* split-row A (_s) and split-row outputs (_so) variants */
-    const char *sfx = a->A2 ? (a->C2 ? "_s_so" : "_s") : (a->C2 ? "_so" : "");
-    static const struct { const char *name, *glu_name, *acc_name; uint32_t bm, bn; } cfg[] = {
-        { "gemm_mx128x128", "gemm_mx128x128_glu", "gemm_mx128x128_acc", 128, 128 },
-        { "gemm_mx64x128", "gemm_mx64x128_glu", "gemm_mx64x128_acc", 64, 128 },
-        { "gemm_mx64x64", "gemm_mx64x64_glu", "gemm_mx64x64_acc", 64, 64 },
-    };
-    int pick_i = -1, last_ok = -1;
-    uint32_t tiles = 0;
     const uint32_t kb = resid ? mx_kblocks(K) : 1;
-    for (int i = 0; i < 3; ++i) {
-        const uint32_t cols = glu ? cfg[i].bn / 2 : cfg[i].bn;
-        if (nout % cols) continue;
-        const uint32_t t = ((M + cfg[i].bm - 1) / cfg[i].bm) * (nout / cols);
-        if (cfg[i].bm == 128 && (M < 512 || a->A2)) continue; /* split rows: one workgroup per CU */
-        last_ok = i;
-        /* two workgroups per CU: the largest tile with at least ~400 workgroups (residual updates:
-         * tiles x K blocks, the split below) was the fastest at every measured shape (448 to 3584
-         * rows, N 1024 to 4096, K 1024 and 4096) */
-        if ((a->A2 ? t * kb : t) >= 400) { pick_i = i; tiles = t; break; }
-    }
-    if (last_ok < 0) return 1;
-    if (g_mx_tile >= 0 && nout % (glu ? cfg[g_mx_tile].bn / 2 : cfg[g_mx_tile].bn) == 0) pick_i = g_mx_tile;
-    if (pick_i >= 0) {
-        const uint32_t cols = glu ? cfg[pick_i].bn / 2 : cfg[pick_i].bn;
-        tiles = ((M + cfg[pick_i].bm - 1) / cfg[pick_i].bm) * (nout / cols);
-    }
-    if (pick_i < 0) {
-        pick_i = last_ok;
-        const uint32_t cols = glu ? cfg[pick_i].bn / 2 : cfg[pick_i].bn;
-        tiles = ((M + cfg[pick_i].bm - 1) / cfg[pick_i].bm) * (nout / cols);
-    }
+    const mx_tile_t *t = mx_pick(!a->A2, M, nout, K, glu, g_split == 0 ? 1 : kb);
+    if (!t) return 1;
+    const uint32_t tiles = mx_tiles(t, M, nout, glu);
     uint32_t kz = 1;
     a->kblocks = 1;
     if (resid) {
-        a->kblocks = mx_kblocks(K);
-        /* split below ~400 tiles (measured on 64 x 64 tiles: about 448 workgroups at 448 rows) */
-        if (a->kblocks > 1 && (g_split == 1 || (g_split < 0 && tiles < 400))) kz = a->kblocks;
+        a->kblocks = kb;
+        /* split-row A: always (a block of 1024 is a workgroup's whole K loop elsewhere too; at 3584 rows
+         * FF down takes 63 us in four blocks against 67-79 unsplit, its four partial rows cost the
+         * LayerNorm that folds them 6 us more).  f32 A: below ~400 tiles */
+        if (kb > 1 && (g_split == 1 || (g_split < 0 && (a->A2 || tiles < 400)))) kz = kb;
         const size_t need = (size_t)kz * M * nout;
         if (sc && sc->ws) {
             /* a fixed region too small for the split may still hold the unsplit partial rows (same
@@ -214,16 +239,25 @@ static int launch_mx_s(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint3
         pend->nparts = kz;
         pend->alpha = a->alpha;
     }
-    const uint32_t tm = (M + cfg[pick_i].bm - 1) / cfg[pick_i].bm;
+    const uint32_t tm = (M + t->bm - 1) / t->bm;
     a->splits = kz;
     /* at most 8 row tiles per group: an XCD's 64 resident workgroups then cover about 8 row tiles x 8
      * column tiles, whose A panels stay in its L2 while the weight columns stream past (at 3584
      * rows: L2 fetch -18% on FF up, -12% on QKV against 14-row groups; 2-4% faster) */
     a->group_m = tm <= 8 ? tm : 8;
     const uint32_t total = tiles * kz, per = (total + 7) / 8;
-    char name[40];
-    snprintf(name, sizeof name, "%s%s", resid ? cfg[pick_i].acc_name : glu ? cfg[pick_i].glu_name : cfg[pick_i].name, sfx);
-    return gpu_launch(g, name, a, sizeof *a, 8 * per, 1, 1, 256, 1, 1);
+    if (total < 65536) {
+        const uint32_t last = tm % a->group_m;
+        a->tm = tm;
+        a->rc_mn = recip32(tiles);
+        a->rc_grp = recip32(a->group_m * (tiles / tm));
+        a->rc_gm = recip32(a->group_m);
+        a->rc_last = recip32(last ? last : a->group_m);
+    }
+    char name[40]; /* split-row A (_s) and split-row outputs (_so) variants */
+    snprintf(name, sizeof name, "gemm_mx%s%s%s%s", t->tile, resid ? "_acc" : glu ? "_glu" : "", a->A2 ? "_s" : "",
+             a->C2 ? "_so" : "");
+    return gpu_launch(g, name, a, sizeof *a, 8 * per, 1, 1, MX_THREADS, 1, 1);
 }
 
 static int launch_mx(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid) {
@@ -255,7 +289,7 @@ static int gemm_split_core(gpu_t *g, const float *A, const uint16_t *A2, uint32_
     if (!M) return 0;
     const int glu = act == NK_ACT_GLU;
     const uint32_t nout = glu ? N / 2 : N;
-    if (!N || !K || (glu && (N & 1)) || K % 32 || (A2 && K % NK_MX_KS_SPLIT) || !A == !A2 || !C == !C2)
+    if (!N || !K || (glu && (N & 1)) || K % 32 || (A2 && K % NK_MX_KS) || !A == !A2 || !C == !C2)
         return bad(g, "gemm_split: one A form, one C form, K % 32 == 0 (K % 64 == 0 with split-row A)");
     if (!aligned16(W) || ldw % 8 || K > ldw) return bad(g, "gemm_split: W 16-byte aligned, ldw % 8 == 0, K <= ldw");
     if (A ? (!aligned16(A) || lda % 4 || K > lda) : (!aligned16(A2) || lda % 8 || 2 * K > lda))
@@ -320,7 +354,7 @@ int nk_gemm_argmax_rows(gpu_t *g, const float *A, uint32_t lda, const uint16_t *
     const uint32_t tm = (M + 63) / 64, tiles = tm * (N / 64), per = (tiles + 7) / 8;
     a.group_m = tm <= 8 ? tm : 8;
     gpu_next_flops(g, 2.0 * M * N * K);
-    return gpu_launch(g, "gemm_mx64x64_argmax", &a, sizeof a, 8 * per, 1, 1, 256, 1, 1);
+    return gpu_launch(g, "gemm_mx64x64_argmax", &a, sizeof a, 8 * per, 1, 1, MX_THREADS, 1, 1);
 }
 
 /* The GEMM with an optional LayerNorm prologue on A.  The weight-streaming GEMV (K <= 1024) and the

@@ -28,7 +28,7 @@ typedef uint16_t u16;
 
 /* Row and chunk limits.  One wavefront is 64 lanes on CDNA4. */
 #define NK_WAVE 64
-#define NK_MX_KS_SPLIT 64       /* K step of the many-row kernels on split-row A (K % this == 0)  */
+#define NK_MX_KS 64             /* K step of the many-row kernels (split-row A: K % this == 0)      */
 #define NK_FEW_ROWS 16          /* GEMMs with M <= 16 use the weight-streaming kernels            */
 #define NK_ATT_MAX_L 128        /* attention window limit (reference ATT_MAX_L 80; 56 + 16 + 2)    */
 #define NK_DEC_MAX_BATCH 16     /* joint rows per decoder round trip (reference DEC_MAX_BATCH)    */
@@ -86,6 +86,11 @@ typedef struct {
     float *fold_out;
     u32 fold_n;
     float fold_alpha;
+    /* many-row kernel, tile order without divisions (64-bit products of the tile number with these,
+     * exact below 65536 tiles): reciprocals 2^32 / d rounded up, 0 for d = 1, of the tiles per K block,
+     * the tiles per group of row tiles, the row tiles of a group and of the last group.  tm: row
+     * tiles; 0: not given, the kernel divides (a row count on the device, more tiles) */
+    u32 tm, rc_mn, rc_grp, rc_gm, rc_last, pad3;
 } NkGemmArgs;
 
 typedef struct {
