@@ -354,115 +354,152 @@ extern "C" __global__ __launch_bounds__(512) void attention_rel(const NkAttnArgs
  *   S2 = (Q + v) P^T   [16][96]  six tiles over the chunk's L + c - 1 position rows
  *   score(i, j) = (S1[i][j] + S2[i][c - 1 - i + j]) * scale,  softmax over j < L
  *   O = softmax . V    [16][128] eight tiles
- * The eleven score tiles are spread over the four wavefronts; a lane reads its K or P row (32
- * consecutive dims of the row) straight from global memory and holds its query row's matching 32
- * dims of q + u and q + v in registers (step s of the K loop is dim 32 (lane / 16) + s on both
- * operands).  V goes to LDS by direct loads (granule g of row r at slot g ^ (r % 16), so the
- * column reads of the P.V product are conflict-free); scores and probabilities go through LDS. */
+ * Only the tiles that hold keys or positions of the chunk are computed.
+ *
+ * Bound by reading the K and V windows from HBM (147 MB at 256 chunks of 14 rows, 30 us at the 4.9 TB/s
+ * of a copy), so everything a workgroup reads is in flight at once: wavefronts 0 and 1 take the K
+ * tiles and hold q + u, 2 and 3 the position tiles and hold q + v (one of the two, so that three
+ * tiles' rows fit the registers of three wavefronts per SIMD), and V streams into LDS behind them.  A
+ * lane's four-dim pieces of a row are dims 16 v + 4 (lane / 16) + (0..3), so that the four lanes of a
+ * row read 64 consecutive bytes: with 32 consecutive dims per lane every load touched 64 lines of
+ * which the next seven loads needed the rest, more than the L1 holds.  V granule g of row r is at
+ * slot g ^ (4 (r % 4) + r / 4 % 4), which makes the column reads of the P.V product (rows 4 k .. 4 k + 3)
+ * conflict-free; V is its first operand, so a lane stores four consecutive dims.   Graph-replayed, 8
+ * heads: 23 chunks of 7 rows 10.3 -> 8.6 us, 64 of 7 16.8 -> 13.4, 256 of 14 62.4 -> 53.5 (eight
+ * wavefronts 69.9: every wavefront loads the query rows again). */
 #define ATC_SLD 97 /* score row stride in floats: 96 position columns + 1 */
-extern "C" __global__ __launch_bounds__(256) void attention_rel_chunks(const NkAttnChunkArgs a) {
+extern "C" __global__ __launch_bounds__(256, 3) void attention_rel_chunks(const NkAttnChunkArgs a) {
     __shared__ floatx4 Vs[NK_ATTC_MAX_L * 32];
     __shared__ float S1[16 * ATC_SLD], S2[16 * ATC_SLD];
     static_assert(NK_ATTC_MAX_L == 80 && NK_ATTC_MAX_C <= 16, "tile counts assume 80 keys, 16 query rows");
-    const u32 h = blockIdx.x, ch = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const u32 h = blockIdx.x, ch = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int *cd = a.chunks + 4 * ch;
     const u32 qrow0 = (u32)cd[0], m0 = (u32)cd[1], c = (u32)cd[2], cl = (u32)cd[3];
     const u32 L = cl + c, NP = L + c - 1;
     if (c == 0 || c > NK_ATTC_MAX_C || L > NK_ATTC_MAX_L || L > a.Lmax) return; /* host-checked */
     const u32 off = h * 128;
-    const float *Kg = a.kv + a.D + (u64)(qrow0 - cl) * a.ld + off;
+    /* V rows 0 .. 16 ceil(L / 16) - 1 into LDS, two rows per direct-load instruction (rows past L re-read
+     * row L - 1: finite values, weighted by zero probabilities).  First, so that the compiler's waits
+     * for the loads below, which do not count these, are exact */
     const float *Vg = a.kv + 2 * a.D + (u64)(qrow0 - cl) * a.ld + off;
-    const float *Pg = a.P + (u64)(a.Lmax - L) * a.D + off;
-    /* V rows 0 .. 79 into LDS, two rows per direct-load instruction (rows past L re-read row L - 1:
-     * finite values, weighted by zero probabilities) */
-    for (u32 blk = wave; blk < NK_ATTC_MAX_L / 2; blk += 4) {
-        const u32 p = blk * 64 + lane, r = p >> 5, g = (p & 31) ^ (r & 15), rr = min(r, L - 1);
-        dma16(Vg + (u64)rr * a.ld + 4 * g, (lds_char_t *)&Vs[blk * 64]);
+    const u32 vgroups = (L + 15) / 16;
+    for (u32 blk = wave; blk < 8 * vgroups; blk += 4) {
+        const u32 r = 2 * blk + (lane >> 5), g = (lane & 31) ^ (4 * (r & 3) + ((r >> 2) & 3));
+        dma16(Vg + (u64)min(r, L - 1) * a.ld + 4 * g, (lds_char_t *)&Vs[blk * 64]);
     }
-    /* query row qi = lane % 16 (zero past c), dims 32 kq .. 32 kq + 31 */
+    /* query row qi = lane % 16 (zero past c) */
     const u32 qi = lane & 15, kq = lane >> 4;
-    float qu[32], qv[32];
-    {
-        const bool ok = qi < c;
-        const floatx4 *qp = (const floatx4 *)(a.kv + (u64)(qrow0 + min(qi, c - 1)) * a.ld + off + 32 * kq);
-        const floatx4 *up = (const floatx4 *)(a.bu + off + 32 * kq), *vp = (const floatx4 *)(a.bv + off + 32 * kq);
+    const bool pos = wave >= 2;
+    const u32 n = pos ? NP : L, ld = pos ? a.D : a.ld; /* rows of this wavefront's operand */
+    const float *src = pos ? a.P + (u64)(a.Lmax - L) * a.D + off : a.kv + a.D + (u64)(qrow0 - cl) * a.ld + off;
+    const floatx4 *qp = (const floatx4 *)(a.kv + (u64)(qrow0 + min(qi, c - 1)) * a.ld + off) + kq;
+    const floatx4 *wp = (const floatx4 *)((pos ? a.bv : a.bu) + off) + kq;
+    floatx4 q[8], b[3][8];
 #pragma unroll
-        for (int v4 = 0; v4 < 8; ++v4) {
-            const floatx4 q = qp[v4], u = up[v4], w = vp[v4];
+    for (int v = 0; v < 8; ++v) q[v] = qp[4 * v];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                qu[4 * v4 + e] = ok ? q[e] + u[e] : 0.0f;
-                qv[4 * v4 + e] = ok ? q[e] + w[e] : 0.0f;
-            }
+    for (int v = 0; v < 8; ++v) {
+        const floatx4 w = wp[4 * v];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[v][e] = qi < c ? q[v][e] + w[e] : 0.0f;
+    }
+    /* this wavefront's tiles: 16-row tiles wave % 2, + 2, + 4 (rows past the last re-read it) */
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        const u32 col0 = 16 * ((wave & 1) + 2 * t);
+        if (t < 2 || col0 < n) {
+            const floatx4 *bp = (const floatx4 *)(src + (u64)min(col0 + qi, n - 1) * ld) + kq;
+#pragma unroll
+            for (int v = 0; v < 8; ++v) b[t][v] = bp[4 * v];
         }
     }
-    /* score tiles: T < 5 content (K rows 16 T ..), T >= 5 position (P rows 16 (T - 5) ..) */
-    for (u32 T = wave; T < 11; T += 4) {
-        const bool pos = T >= 5;
-        const u32 col0 = (pos ? T - 5 : T) * 16, row = col0 + qi;
-        const floatx4 *src = (const floatx4 *)((pos ? Pg + (u64)min(row, NP - 1) * a.D : Kg + (u64)min(row, L - 1) * a.ld) +
-                                               32 * kq);
-        float b[32];
+    float *S = pos ? S2 : S1;
 #pragma unroll
-        for (int v4 = 0; v4 < 8; ++v4) {
-            const floatx4 x = src[v4];
+    for (int t = 0; t < 3; ++t) {
+        const u32 col0 = 16 * ((wave & 1) + 2 * t);
+        if (col0 < n) {
+            floatx4 acc = { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-            for (int e = 0; e < 4; ++e) b[4 * v4 + e] = x[e];
-        }
-        floatx4 acc = { 0.f, 0.f, 0.f, 0.f };
-        if (pos) {
+            for (int v = 0; v < 8; ++v)
 #pragma unroll
-            for (int k = 0; k < 32; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[k], b[k], acc, 0, 0, 0);
-        } else {
+                for (int e = 0; e < 4; ++e)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[v][e], b[t][v][e], acc, 0, 0, 0);
 #pragma unroll
-            for (int k = 0; k < 32; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qu[k], b[k], acc, 0, 0, 0);
-        }
-        float *S = pos ? S2 : S1;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[(4 * kq + r) * ATC_SLD + col0 + qi] = acc[r];
-    }
-    wait_vm_lgkm<0>();
-    barrier_mem();
-    /* scores and softmax: wavefront w takes rows w, w + 4, ...; lane takes keys lane, lane + 64;
-     * the probabilities replace S1 (zero for rows past c and keys past L) */
-    for (u32 i = wave; i < 16; i += 4) {
-        const u32 j0 = lane, j1 = lane + 64;
-        if (i < c) {
-            const bool v0 = j0 < L, v1 = j1 < L;
-            const float s0 = v0 ? (S1[i * ATC_SLD + j0] + S2[i * ATC_SLD + (c - 1 - i + j0)]) * a.scale : -INFINITY;
-            const float s1 = v1 ? (S1[i * ATC_SLD + j1] + S2[i * ATC_SLD + (v1 ? c - 1 - i + j1 : 0)]) * a.scale : -INFINITY;
-            const float mx = wave_max(fmaxf(s0, s1));
-            const float e0 = v0 ? expf(s0 - mx) : 0.0f, e1 = v1 ? expf(s1 - mx) : 0.0f;
-            const float sum = wave_sum(e0 + e1);
-            S1[i * ATC_SLD + j0] = e0 / sum;
-            if (j1 < NK_ATTC_MAX_L) S1[i * ATC_SLD + j1] = e1 / sum;
-        } else {
-            S1[i * ATC_SLD + j0] = 0.0f;
-            if (j1 < NK_ATTC_MAX_L) S1[i * ATC_SLD + j1] = 0.0f;
+            for (int r = 0; r < 4; ++r) S[(4 * kq + r) * ATC_SLD + col0 + qi] = acc[r];
         }
     }
     lds_barrier();
-    /* O = P V: wavefront w takes output column tiles w and w + 4; step s of the K loop is key
-     * 20 (lane / 16) + s on both operands */
-    for (u32 dt = wave; dt < 8; dt += 4) {
-        const u32 d = dt * 16 + qi, gq = d >> 2, e = d & 3;
-        floatx4 acc = { 0.f, 0.f, 0.f, 0.f };
+    /* scores and softmax: wavefront w takes rows w, w + 4, ...; lane takes keys lane, lane + 64;
+     * the probabilities replace S1 (zero for rows past c and keys past L) */
+    const bool v0 = lane < L, v1 = lane + 64 < L;
+    const u32 j1 = min(lane + 64, (u32)NK_ATTC_MAX_L - 1);
 #pragma unroll
-        for (u32 k = 0; k < NK_ATTC_MAX_L / 4; ++k) {
-            const u32 j = (NK_ATTC_MAX_L / 4) * kq + k;
-            const float pa = S1[qi * ATC_SLD + j];
-            const float vb = ((const float *)&Vs[j * 32 + (gq ^ (j & 15))])[e];
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, vb, acc, 0, 0, 0);
-        }
+    for (int r = 0; r < 4; r += 2) { /* two rows at a time: their reductions overlap */
+        float p[2][2] = { { 0.f, 0.f }, { 0.f, 0.f } };
+        if (wave + 4 * r < c) {
+            float mx[2], sum[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const u32 i = 4 * kq + r;
-            if (i < c) {
-                if (a.Os) store_split1(a.Os + (u64)(m0 + i) * 2 * a.D, a.D, off + d, acc[r]);
-                else a.O[(u64)(m0 + i) * a.D + off + d] = acc[r];
+            for (int k = 0; k < 2; ++k) {
+                /* a second row past c: row c - 1, read in vain (another wavefront may be replacing it) */
+                const u32 i = min(wave + 4 * (r + k), c - 1), d = c - 1 - i; /* d < 16 */
+                const float *x = S1 + i * ATC_SLD, *y = S2 + i * ATC_SLD + d;
+                const float t0 = (x[lane] + y[lane]) * a.scale, t1 = (x[j1] + y[j1]) * a.scale;
+                p[k][0] = v0 ? t0 : -INFINITY;
+                p[k][1] = v1 ? t1 : -INFINITY;
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) mx[k] = wmax(fmaxf(p[k][0], p[k][1]));
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                p[k][0] = v0 ? expf(p[k][0] - mx[k]) : 0.0f;
+                p[k][1] = v1 ? expf(p[k][1] - mx[k]) : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) sum[k] = wsum(p[k][0] + p[k][1]); /* >= 1 */
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const bool in = wave + 4 * (r + k) < c;
+                p[k][0] = in ? div_ge1(p[k][0], sum[k]) : 0.0f;
+                p[k][1] = in ? div_ge1(p[k][1], sum[k]) : 0.0f;
             }
         }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const u32 i = wave + 4 * (r + k);
+            S1[i * ATC_SLD + lane] = p[k][0];
+            if (lane + 64 < NK_ATTC_MAX_L) S1[i * ATC_SLD + lane + 64] = p[k][1];
+        }
     }
+    wait_vm_lgkm<0>(); /* V is in LDS */
+    barrier_mem();
+    /* O = P V: wavefront w takes output column tiles w and w + 4; step k is keys 4 k + lane / 16, four
+     * steps' operands read at a time */
+    floatx4 o[2] = { { 0.f, 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f, 0.f } };
+    for (u32 g = 0; g < vgroups; ++g) {
+        float pa[4], vb[2][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32 j = 16 * g + 4 * k + kq;
+            pa[k] = S1[qi * ATC_SLD + j];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                vb[t][k] = ((const float *)&Vs[j * 32 + ((4 * (wave + 4 * t) + (qi >> 2)) ^ (4 * kq + k))])[qi & 3];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vb[t][k], pa[k], o[t], 0, 0, 0);
+    }
+    if (qi < c)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const u32 d = off + 16 * (wave + 4 * t) + 4 * kq;
+            if (a.Os) store_split4(a.Os + (u64)(m0 + qi) * 2 * a.D, a.D, d, make_float4(o[t][0], o[t][1], o[t][2], o[t][3]));
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a.O[(u64)(m0 + qi) * a.D + d + e] = o[t][e];
+        }
 }
 
 /* Causal depthwise conv (9 taps: 8 history rows + the row itself, no bias) + LN + SiLU, one
