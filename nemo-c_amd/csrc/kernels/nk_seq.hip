@@ -548,3 +548,103 @@ extern "C" __global__ __launch_bounds__(256) void dwconv_ln_silu(const NkDwArgs 
             else y[tid + k * 256] = o;
         }
 }
+
+/* dwconv_ln_silu for the rows of many streams (row table, D <= 1024): DWR table rows per workgroup.  A
+ * row's own workgroup spends its time on the taps (36 floats per thread at a stride of 144 bytes: nine
+ * loads of ~72 lines each) and on eight barriers after one memory round trip; here the taps come
+ * through LDS by direct loads in whole lines, once for all rows, rows on consecutive cache rows (one
+ * chunk's) read rows + 8 input rows instead of 9 each, and the two LayerNorm reductions of all rows
+ * share two barriers.  Other tables (several chunks in one workgroup) load each row's nine input rows,
+ * one row ahead of its sums; a row's sums are the same either way.  3584
+ * rows (256 chunks of 14), graph-replayed: 25.6 -> 16.9 us, of which 7.6 are one workgroup's latency
+ * and a launch (37 MB read and written: 7.6 us at the rate of a copy). */
+#define DWR NK_DW_ROWS
+extern "C" __global__ __launch_bounds__(256) void dwconv_rows(const NkDwArgs a) {
+    __shared__ uint4 taps[(1024 * DW_TAPS * 4 + 1008) / 16];
+    __shared__ float red[2][DWR][4];
+    const u32 m = blockIdx.x * DWR, tid = threadIdx.x, lane = tid & 63, D4 = a.D >> 2;
+    const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = min(a.c - m, (u32)DWR);
+    const int cache_row = a.rows[4 * (u64)min(m + lane, a.c - 1)]; /* lane r: of row m + r */
+    const u32 tb = a.D * DW_TAPS * 4; /* bytes of taps */
+    for (u32 p = wave; p * 1024 < tb; p += 4)
+        dma16((const char *)a.W + min(p * 1024 + lane * 16, tb - 16), (lds_char_t *)taps + p * 1024);
+    const u32 c4 = min(tid, D4 - 1);
+    const float4 g = ((const float4 *)a.g)[c4], b = ((const float4 *)a.b)[c4];
+    const int row0 = __builtin_amdgcn_readlane(cache_row, 0);
+    const bool run = __all(lane >= n || cache_row == row0 + (int)lane);
+    const float *din = a.din - (DW_TAPS - 1) * (long long)a.D + 4 * c4;
+    float wf[4 * DW_TAPS]; /* channel e, tap q of this thread's four channels is element 9 e + q */
+    auto read_taps = [&] {
+        wait_vm_lgkm<0>();
+        barrier_mem();
+#pragma unroll
+        for (int q = 0; q < DW_TAPS; ++q) {
+            const uint4 w = taps[c4 * DW_TAPS + q];
+            wf[4 * q] = __uint_as_float(w.x), wf[4 * q + 1] = __uint_as_float(w.y);
+            wf[4 * q + 2] = __uint_as_float(w.z), wf[4 * q + 3] = __uint_as_float(w.w);
+        }
+    };
+    float v[DWR][4];
+    auto conv = [&](float (&o)[4], const float4 *x) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < DW_TAPS; ++q) {
+            o[0] += wf[0 * DW_TAPS + q] * x[q].x;
+            o[1] += wf[1 * DW_TAPS + q] * x[q].y;
+            o[2] += wf[2 * DW_TAPS + q] * x[q].z;
+            o[3] += wf[3 * DW_TAPS + q] * x[q].w;
+        }
+    };
+    if (run) {
+        float4 x[DWR + DW_TAPS - 1];
+#pragma unroll
+        for (int j = 0; j < DWR + DW_TAPS - 1; ++j)
+            x[j] = *(const float4 *)(din + ((long long)row0 + min((u32)j, n + DW_TAPS - 2)) * a.D);
+        read_taps();
+#pragma unroll
+        for (int r = 0; r < DWR; ++r) conv(v[r], x + r);
+    } else {
+        float4 x[2][DW_TAPS];
+        auto load = [&](int r, int z) {
+            const float *p = din + (long long)__builtin_amdgcn_readlane(cache_row, min((u32)r, n - 1)) * a.D;
+#pragma unroll
+            for (int q = 0; q < DW_TAPS; ++q) x[z][q] = *(const float4 *)(p + (u64)q * a.D);
+        };
+        load(0, 0);
+        load(1, 1);
+        read_taps();
+#pragma unroll
+        for (int r = 0; r < DWR; ++r) {
+            conv(v[r], x[r & 1]);
+            if (r + 2 < DWR) load(r + 2, r & 1);
+        }
+    }
+    /* LayerNorm of the rows (those past n repeat row n - 1), dwconv_ln_silu's sums in its order */
+#pragma unroll
+    for (int r = 0; r < DWR; ++r) {
+        const float s = wave_sum(tid < D4 ? ((v[r][0] + v[r][1]) + v[r][2]) + v[r][3] : 0.0f);
+        if (lane == 0) red[0][r][wave] = s;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < DWR; ++r) {
+        const float mean = (((red[0][r][0] + red[0][r][1]) + red[0][r][2]) + red[0][r][3]) / (float)a.D;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[r][e] -= mean;
+        const float s = wave_sum(tid < D4 ? ((v[r][0] * v[r][0] + v[r][1] * v[r][1]) + v[r][2] * v[r][2]) + v[r][3] * v[r][3] : 0.0f);
+        if (lane == 0) red[1][r][wave] = s;
+    }
+    lds_barrier();
+    if (tid >= D4) return;
+#pragma unroll
+    for (int r = 0; r < DWR; ++r)
+        if ((u32)r < n) {
+            const float var = ((red[1][r][0] + red[1][r][1]) + red[1][r][2]) + red[1][r][3];
+            const float inv = 1.0f / sqrtf(var / (float)a.D + a.eps);
+            const float4 o = make_float4(silu_f(v[r][0] * inv * g.x + b.x), silu_f(v[r][1] * inv * g.y + b.y),
+                                         silu_f(v[r][2] * inv * g.z + b.z), silu_f(v[r][3] * inv * g.w + b.w));
+            if (a.Ys) store_split4(a.Ys + (u64)(m + r) * 2 * a.D, a.D, 4 * tid, o);
+            else *(float4 *)(a.Y + (u64)(m + r) * a.D + 4 * tid) = o;
+        }
+}
