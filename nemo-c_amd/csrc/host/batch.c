@@ -402,18 +402,26 @@ static int bdec_state_reset(nemoasr_batch_t *b, int s) {
 }
 
 /* device state of one stream back to that after open: zero LSTM states (and so zero hidden halves
- * of layer 0) and conv history */
+ * of layer 0) and conv history, the greedy loop's state */
 static int stream_zero_device(nemoasr_batch_t *b, int s) {
     const size_t D = (size_t)b->m->cfg.d_model, P = (size_t)b->P;
-    const size_t n = (size_t)b->conv_left * D > 8 * P ? (size_t)b->conv_left * D : 8 * P;
-    float *z = calloc(n, sizeof(float));
-    int rc = gpu_upload(b->g, (float *)gpu_buf_dptr(b->hc) + (size_t)s * 8 * P, z, 8 * P * sizeof(float));
-    rc |= gpu_upload(b->g, (float *)gpu_buf_dptr(b->pre0) + (size_t)s * 8 * P, z, 8 * P * sizeof(float));
-    for (int l = 0; l < b->m->cfg.n_layers; ++l)
-        rc |= gpu_upload(b->g, (float *)gpu_buf_dptr(b->din) + (size_t)l * b->din_lstride + (size_t)s * b->cap_rows * D, z,
-                         (size_t)b->conv_left * D * sizeof(float));
-    free(z);
-    return rc | bdec_state_reset(b, s);
+    NkBDecStream x;
+    memset(&x, 0, sizeof x);
+    x.last_token = b->m->cfg.blank_id;
+    NkResetArgs a;
+    memset(&a, 0, sizeof a);
+    a.base = (float *)gpu_buf_dptr(b->din) + (size_t)s * b->cap_rows * D;
+    a.stride = b->din_lstride;
+    a.nbuf = (uint32_t)b->m->cfg.n_layers;
+    a.n = (uint32_t)((size_t)b->conv_left * D);
+    a.z0 = (float *)gpu_buf_dptr(b->hc) + (size_t)s * 8 * P;
+    a.z1 = (float *)gpu_buf_dptr(b->pre0) + (size_t)s * 8 * P;
+    a.zn = (uint32_t)(8 * P);
+    a.st = (int *)((NkBDecStream *)gpu_buf_dptr(b->bst) + s);
+    a.words = sizeof x / sizeof(int);
+    _Static_assert(sizeof x <= sizeof a.val && sizeof x % sizeof(int) == 0, "stream state fits the reset arguments");
+    memcpy(a.val, &x, sizeof x);
+    return nk_stream_reset(b->g, &a);
 }
 
 nemoasr_batch_t *nemoasr_batch_open(const char *model_dir, const char *language, int latency_ms, int n_streams,

@@ -96,15 +96,19 @@ void decoder_destroy(decoder_t *d) {
 /* src/decoder.c:48-53: zero LSTM state (so Wh0 . h0 is zero too), last token blank, no valid
  * prediction */
 void decoder_reset(decoder_t *d) {
-    const size_t P = (size_t)d->m->cfg.pred_hidden;
-    float *z = calloc(2 * 4 * P, sizeof(float));
-    gpu_upload(d->g, gpu_buf_dptr(d->hc), z, 2 * 4 * P * sizeof(float));
-    gpu_upload(d->g, gpu_buf_dptr(d->pre0), z, 2 * 4 * P * sizeof(float));
-    free(z);
     NkDecState s[2];
     memset(s, 0, sizeof s);
     s[0].last_token = d->m->cfg.blank_id;
-    gpu_upload(d->g, gpu_buf_dptr(d->st), s, sizeof s);
+    NkResetArgs a;
+    memset(&a, 0, sizeof a);
+    a.z0 = gpu_buf_dptr(d->hc);
+    a.z1 = gpu_buf_dptr(d->pre0);
+    a.zn = (uint32_t)(2 * 4 * d->m->cfg.pred_hidden);
+    a.st = gpu_buf_dptr(d->st);
+    a.words = 2 * sizeof(NkDecState) / sizeof(int);
+    _Static_assert(sizeof s <= sizeof a.val, "loop state fits the reset arguments");
+    memcpy(a.val, s, sizeof s);
+    if (a.z0 && a.z1 && a.st) nk_stream_reset(d->g, &a);
 }
 double decoder_last_ms(const decoder_t *d) { return d->last_ms; }
 void decoder_use_graphs(decoder_t *d, int on) {

@@ -216,11 +216,13 @@ void encoder_reset(encoder_t *e) {
     e->closed = 0;
     e->cache_len = 0;
     e->pos = e->conv_left;
-    const size_t D = (size_t)e->m->cfg.d_model;
-    float *z = calloc((size_t)e->conv_left * D, sizeof(float));
-    for (int l = 0; l < e->m->cfg.n_layers; ++l)
-        gpu_upload(e->g, (float *)gpu_buf_dptr(e->din) + (size_t)l * e->din_stride, z, (size_t)e->conv_left * D * sizeof(float));
-    free(z);
+    NkResetArgs a;
+    memset(&a, 0, sizeof a);
+    a.base = gpu_buf_dptr(e->din);
+    a.stride = e->din_stride;
+    a.nbuf = (uint32_t)e->m->cfg.n_layers;
+    a.n = (uint32_t)(e->conv_left * e->m->cfg.d_model);
+    if (a.base) nk_stream_reset(e->g, &a);
     e->d_frames = 0;
 }
 

@@ -14,6 +14,7 @@
  */
 #ifndef NEMO_GPU_H
 #define NEMO_GPU_H
+#include "../kernel_params.h"
 #include <stddef.h>
 #include <stdint.h>
 
@@ -122,6 +123,9 @@ int gpu_many_rows(const gpu_t *g);
 
 /* Number of kernel launches issued since creation (for tests and the launch-count check). */
 uint64_t gpu_launch_count(const gpu_t *g);
+
+/* One launch that puts a stream's device state back to a fresh stream's, waited for (nk.c). */
+int nk_stream_reset(gpu_t *g, const NkResetArgs *a);
 
 #ifdef __cplusplus
 }

@@ -751,6 +751,15 @@ int nk_dwconv_ln_silu_rows_split(gpu_t *g, const float *din_base, const int *row
 
 static uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + 255) / 256); }
 
+/* a stream's device state zeroed and its loop state set (NkResetArgs), waited for */
+int nk_stream_reset(gpu_t *g, const NkResetArgs *a) {
+    const uint32_t n = a->n > a->zn ? a->n : a->zn;
+    if (gpu_begin(g)) return -1;
+    gpu_launch(g, "stream_reset", a, sizeof *a, blocks_for(n > NK_RESET_WORDS ? n : NK_RESET_WORDS), a->nbuf + 1, 1, 256, 1,
+               1);
+    return gpu_end(g, NULL, 0);
+}
+
 /* output columns per workgroup of the subsampling convs: one (every output its own workgroup, one
  * memory round trip) unless the batch has thousands of output positions, then eight (fewer
  * workgroups, the filter taps loaded once for eight columns) */

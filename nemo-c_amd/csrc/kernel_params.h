@@ -275,6 +275,20 @@ typedef struct {
     u32 nbuf, rows, cols, src_row, dst_row, pad;
 } NkCompactArgs;
 
+/* A stream's device state back to a fresh stream's in one launch: n floats zeroed in each of nbuf
+ * buffers `stride` floats apart (the conv histories of the layers), zn floats at z0 and z1 (LSTM
+ * states and stored hidden halves; may be NULL) and `words` words of val stored at st (the greedy
+ * loop's state; may be 0). */
+#define NK_RESET_WORDS 32
+typedef struct {
+    float *base;
+    unsigned long long stride;
+    float *z0, *z1;
+    int *st;
+    u32 nbuf, n, zn, words;
+    int val[NK_RESET_WORDS];
+} NkResetArgs;
+
 /* ---- device-resident greedy RNNT loop -------------------------------------------------------- */
 #define NK_DEC_MAX_TOKENS 256 /* tokens per chunk: at most 16 frames x max_symbols                  */
 #define NK_DEC_GROUPS 40      /* joint workgroups per frame row, 32 vocabulary rows each (V <= 1280) */

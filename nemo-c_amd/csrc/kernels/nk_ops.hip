@@ -246,6 +246,22 @@ extern "C" __global__ __launch_bounds__(256) void compact_rows4(const NkCompactA
     b[(u64)a.dst_row * (a.cols / 4) + idx] = b[(u64)a.src_row * (a.cols / 4) + idx];
 }
 
+/* State of a fresh stream (NkResetArgs); grid = (ceil(max(n, zn) / 256), nbuf + 1), the last y the
+ * decoder's part.  One launch for the copies of a stream's reset: they were 27 small host-to-device
+ * copies of zeros, each waited for (~8 us), 14 of the 51 ms of a pass that resets 64 streams. */
+extern "C" __global__ __launch_bounds__(256) void stream_reset(const NkResetArgs a) {
+    const u32 i = blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.y < a.nbuf) {
+        if (i < a.n) a.base[blockIdx.y * a.stride + i] = 0.0f;
+        return;
+    }
+    if (i < a.zn) {
+        if (a.z0) a.z0[i] = 0.0f;
+        if (a.z1) a.z1[i] = 0.0f;
+    }
+    if (i < a.words) a.st[i] = a.val[i];
+}
+
 /* Strided row copy: rows x cols floats from src (row stride src_ld) to dst (row stride dst_ld).
  * Used for the row select of the subsampled window and for activation dumps. */
 extern "C" __global__ __launch_bounds__(256) void copy2d_f32(const NkCopy2dArgs a) {
