@@ -61,6 +61,12 @@ __device__ __forceinline__ void ln_wave4(floatx4 (&v)[4], const floatx4 (&g)[4],
  * variant, so that they load with the rows (and the parts) without holding registers through the
  * fold. */
 #define FR_FOLD_PARTS 4
+/* LDS row stride of the normalised activations in floats: 16 bytes past 4 KB, so that the 16 rows of
+ * an operand read start in different banks.  With rows 4 KB apart each of a wavefront's eight
+ * ds_read_b128 met a 16-way conflict.
+ * Graph-replayed, FF up / QKV with four pending parts: 7 rows 9.34 -> 8.89, 8.31 -> 7.91 us; 14 rows
+ * 11.04 -> 10.63, 9.29 -> 8.88 us; without parts FF up 6.56 -> 6.11, 7.14 -> 6.69 us. */
+#define FR_LD 1028
 /* PK (GLU only): a workgroup owns 8 output pairs, whose value and gate weight rows share one
  * 16-column B operand (columns 0-7 values, 8-15 gates), so there is one MFMA pair per step and
  * twice the workgroups; the epilogue takes each gate sum from lane ^ 8.  Every output's value and
@@ -219,7 +225,7 @@ __device__ __forceinline__ void fr_impl(const NkGemmArgs &a, float *sA, floatx4 
                     for (int j = 0; j < 4; ++j) ((floatx4 *)(a.ln_out + (u64)r * a.lda))[lane + 64 * j] = v[i][j];
                 if (a.ln_mode == 2) ln_wave4(v[i], g2, b2, D, a.ln_eps);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) ((floatx4 *)(sA + (u64)r * 1024))[lane + 64 * j] = v[i][j];
+                for (int j = 0; j < 4; ++j) ((floatx4 *)(sA + (u64)r * FR_LD))[lane + 64 * j] = v[i][j];
             }
         }
         lds_barrier();
@@ -232,7 +238,7 @@ __device__ __forceinline__ void fr_impl(const NkGemmArgs &a, float *sA, floatx4 
         if ((u32)s < ns) {
             uint4 ah, al;
             if constexpr (LNA) {
-                const float *sp = sA + (u64)m * 1024 + (sb + s) * 32 + kq;
+                const float *sp = sA + (u64)m * FR_LD + (sb + s) * 32 + kq;
                 const floatx4 p = *(const floatx4 *)sp, q = *(const floatx4 *)(sp + 4);
                 const float xs[8] = { p[0], p[1], p[2], p[3], q[0], q[1], q[2], q[3] };
                 split8(xs, ah, al);
@@ -311,7 +317,7 @@ GEMM_FR(gemm_fr_glu_w4s8, 4, 8, true)
  * with the pending-update fold */
 #define GEMM_FR_LN(NAME, GLU, FOLD)                                                                      \
     extern "C" __global__ __launch_bounds__(512) void NAME(const NkGemmArgs a) {                         \
-        __shared__ float sA[16 * 1024];                                                                  \
+        __shared__ float sA[16 * FR_LD];                                                                  \
         __shared__ floatx4 sred[8 * 64];                                                                 \
         __shared__ floatx4 sP[1024];                                                                     \
         fr_impl<8, 4, true, GLU, FOLD, GLU>(a, sA, sred, sP);                                            \
