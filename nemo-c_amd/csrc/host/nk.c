@@ -157,19 +157,18 @@ static uint32_t recip32(uint32_t d) { return d > 1 ? (uint32_t)(((1ull << 32) + 
  * work per step), fitted to the subsampling's GEMMs and joint.enc at 64 to 40128 rows. */
 typedef struct {
     const char *tile;
-    uint16_t bm, bn, slots;
+    uint16_t bm, bn, slots, threads, glu_threads;
     struct { float fix, step, fix1, step1; } us[2]; /* fix 0: not built for this form */
 } mx_tile_t;
 static const mx_tile_t mx_tile[] = { /* in the order of nk_gemm_mx_tile's numbers */
-    { "128x256", 128, 256, 256, { { 5.0f, 1.45f, 5.0f, 1.45f }, { 0 } } },
-    { "64x128", 64, 128, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
-    { "64x64", 64, 64, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
-    { "32x64", 32, 64, 256, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
-    { "32x32", 32, 32, 256, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
-    { "64x128d", 64, 128, 256, { { 2.5f, 0.63f, 2.5f, 0.63f }, { 0 } } },
+    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.45f, 5.0f, 1.45f }, { 0 } } },
+    { "64x128", 64, 128, 512, 512, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
+    { "64x64", 64, 64, 512, 512, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
+    { "32x64", 32, 64, 256, 512, 512, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
+    { "32x32", 32, 32, 256, 512, 512, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
+    { "64x128d", 64, 128, 256, 768, 512, { { 2.2f, 0.57f, 2.2f, 0.57f }, { 0 } } },
 };
 #define MX_TILES ((int)(sizeof mx_tile / sizeof *mx_tile))
-#define MX_THREADS 512 /* every kernel: 8 computing wavefronts, or 4 that compute and 4 that load */
 
 static uint32_t mx_tiles(const mx_tile_t *t, uint32_t M, uint32_t nout, int glu) {
     const uint32_t cols = glu ? t->bn / 2u : t->bn;
@@ -257,7 +256,7 @@ static int launch_mx_s(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint3
     char name[40]; /* split-row A (_s) and split-row outputs (_so) variants */
     snprintf(name, sizeof name, "gemm_mx%s%s%s%s", t->tile, resid ? "_acc" : glu ? "_glu" : "", a->A2 ? "_s" : "",
              a->C2 ? "_so" : "");
-    return gpu_launch(g, name, a, sizeof *a, 8 * per, 1, 1, MX_THREADS, 1, 1);
+    return gpu_launch(g, name, a, sizeof *a, 8 * per, 1, 1, glu ? t->glu_threads : t->threads, 1, 1);
 }
 
 static int launch_mx(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid) {
@@ -354,7 +353,7 @@ int nk_gemm_argmax_rows(gpu_t *g, const float *A, uint32_t lda, const uint16_t *
     const uint32_t tm = (M + 63) / 64, tiles = tm * (N / 64), per = (tiles + 7) / 8;
     a.group_m = tm <= 8 ? tm : 8;
     gpu_next_flops(g, 2.0 * M * N * K);
-    return gpu_launch(g, "gemm_mx64x64_argmax", &a, sizeof a, 8 * per, 1, 1, MX_THREADS, 1, 1);
+    return gpu_launch(g, "gemm_mx64x64_argmax", &a, sizeof a, 8 * per, 1, 1, 512, 1, 1);
 }
 
 /* The GEMM with an optional LayerNorm prologue on A.  The weight-streaming GEMV (K <= 1024) and the

@@ -18,7 +18,7 @@
  * instruction (four wavefronts on a CU stream 138 GB/s, eight 217, sixteen 323, measured from L2)
  * and then waits for its fragment reads.
  *   - PW = 4: four more wavefronts only load, so the computing ones never issue a DMA; 18 rows,
- *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 14.2, FF down 13.8 -> 11.8.  All tiles but one.
+ *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 13.4, FF down 13.8 -> 12.1.  All tiles but one.
  *   - PW = 0: 128x256 computed and loaded by eight wavefronts (two per SIMD, 198 VGPRs each: no room
  *     for loaders), half the staged bytes per MFMA of 64x128: its steps of 1.5 us run at 1.2 PFLOP/s
  *     issued, the rate of a large library product here; 3584 rows, FF up 81.7 -> 68.6 us, pw1
@@ -417,7 +417,8 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
  * are more than 256 workgroups.  64x128d (four stages), 32x64 and 32x32 take a CU each, with nearly
  * all of a 1024-column K loop's loads in flight at once: for launches of up to 256 workgroups, whose
  * time is the latency of one.  At 18 rows FF up takes 6.5 us on 32x32 tiles, 7.3 on 32x64, 8.7 on
- * 64x64; at 448 rows 14.2 on 64x128d, 14.7 on 64x64, 16.8 on 64x128.  The host chooses by a cost per
+ * 64x64; at 448 rows 13.6 on 64x128d (eight computing wavefronts, which share the epilogue; with four 15.0), 14.5
+ * on 64x64, 16.8 on 64x128.  The host chooses by a cost per
  * round (mx_tile in csrc/host/nk.c).  Second launch bound: wavefronts per SIMD where two workgroups
  * fit a CU's LDS. */
 #define GEMM_MX(NAME, BM, BN, WGM, WGN, PW, NS, GLU, EPI, AS, OS)                                         \
@@ -443,7 +444,8 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
 #define GEMM_MX_FF(...) GEMM_MX_F(__VA_ARGS__) GEMM_MX_FG(__VA_ARGS__)
 GEMM_MX_SS(128x256, 128, 256, 2, 4, 0, 2)
 GEMM_MX_SS(64x128, 64, 128, 2, 2, 4, 2)
-GEMM_MX_SS(64x128d, 64, 128, 2, 2, 4, 4)
+GEMM_MX_S(64x128d, 64, 128, 2, 4, 4, 4)
+GEMM_MX_SG(64x128d, 64, 128, 2, 2, 4, 4)
 GEMM_MX_SS(64x64, 64, 64, 2, 2, 4, 3)
 GEMM_MX_SS(32x64, 32, 64, 2, 2, 4, 9)
 GEMM_MX_S(32x32, 32, 32, 2, 2, 4, 12)
