@@ -13,7 +13,7 @@ static int g_mx_tile = -1; /* many-row tile: -1 by estimate, else an index of mx
 
 int nk_gemm_mx_tile(int t) {
     const int prev = g_mx_tile;
-    g_mx_tile = t < 0 || t > 5 ? -1 : t;
+    g_mx_tile = t < 0 || t > 6 ? -1 : t;
     return prev;
 }
 
@@ -161,12 +161,13 @@ typedef struct {
     struct { float fix, step, fix1, step1; } us[2]; /* fix 0: not built for this form */
 } mx_tile_t;
 static const mx_tile_t mx_tile[] = { /* in the order of nk_gemm_mx_tile's numbers */
-    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.45f, 5.0f, 1.45f }, { 0 } } },
+    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.70f, 5.0f, 1.50f }, { 0 } } },
     { "64x128", 64, 128, 512, 512, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
     { "64x64", 64, 64, 512, 512, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
     { "32x64", 32, 64, 256, 512, 512, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
     { "32x32", 32, 32, 256, 512, 512, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
-    { "64x128d", 64, 128, 256, 768, 512, { { 2.2f, 0.57f, 2.2f, 0.57f }, { 0 } } },
+    { "64x128d", 64, 128, 256, 768, 512, { { 3.0f, 0.58f, 2.2f, 0.57f }, { 0 } } },
+    { "64x128u", 64, 128, 512, 256, 0, { { 3.5f, 0.95f, 3.0f, 0.76f }, { 0 } } }, /* residual updates, K not split */
 };
 #define MX_TILES ((int)(sizeof mx_tile / sizeof *mx_tile))
 
@@ -176,23 +177,34 @@ static uint32_t mx_tiles(const mx_tile_t *t, uint32_t M, uint32_t nout, int glu)
     return (M + t->bm - 1) / t->bm * (nout / cols);
 }
 
-/* the tile of an (M, nout, K) GEMM, NULL when none divides the output columns; kb: K blocks that may
- * run as workgroups of their own (residual updates) */
-static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, int glu, uint32_t kb) {
+/* The tile of an (M, nout, K) GEMM, NULL when none divides the output columns, and whether its kb K
+ * blocks (residual updates) run as workgroups of their own (*kz = kb) or one after another (1): the
+ * least estimated time, with what each partial row after the first costs the LayerNorm that folds it
+ * (3584 x 1024, three more: 6.4 us).  One after another they run on the kernel that keeps their sum in
+ * registers (FF down with its LayerNorm at 3584 rows: 72 us, 77 split on 128x256), elsewhere only when
+ * asked to. */
+static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid, uint32_t kb,
+                                uint32_t *kz) {
     const mx_tile_t *best = NULL;
     float least = 0;
     if (nout % (glu ? 32 : 64)) return NULL;
     for (int i = 0; i < MX_TILES; ++i) {
         const mx_tile_t *t = &mx_tile[i];
-        const uint32_t tiles = t->us[f32].fix > 0 ? mx_tiles(t, M, nout, glu) : 0;
+        const int unsplit = !t->glu_threads;
+        const uint32_t tiles = t->us[f32].fix > 0 && (!unsplit || (resid && g_split != 1)) ? mx_tiles(t, M, nout, glu) : 0;
         if (!tiles) continue;
-        if (i == g_mx_tile) return t;
-        const uint32_t wgs = tiles * kb;
-        const float steps = (float)(K / kb) / NK_MX_KS;
-        const float us = wgs <= 256 ? t->us[f32].fix1 + t->us[f32].step1 * steps
-                                    : (float)((wgs + t->slots - 1) / t->slots) * (t->us[f32].fix + t->us[f32].step * steps);
+        const uint32_t z = unsplit || g_split == 0 || (f32 && g_split < 0 && tiles >= 400) ? 1 : kb, wgs = tiles * z;
+        if (i == g_mx_tile) {
+            *kz = z;
+            return t;
+        }
+        const float steps = (float)(K / z) / NK_MX_KS;
+        const float us = (wgs <= 256 ? t->us[f32].fix1 + t->us[f32].step1 * steps
+                                     : (float)((wgs + t->slots - 1) / t->slots) * (t->us[f32].fix + t->us[f32].step * steps)) +
+                         (float)(z - 1) * (float)M * (float)nout * (4 / 6.8e6f);
         if (!best || us < least) {
             best = t;
+            *kz = z;
             least = us;
         }
     }
@@ -200,25 +212,21 @@ static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, 
 }
 
 /* Many-row GEMM.  Residual updates (accumulate, no bias, no activation, no row map) run on the _acc
- * kernels: their K sum is blocked (mx_kblocks), and split-row ones run one K block per workgroup (f32
- * ones below 400 tiles); the sums go to partial rows in the scratch (nparts of them, same bits either
- * way); *pend then describes the update still to apply (NkFoldArgs).
+ * kernels: their K sum is blocked (mx_kblocks), the blocks run as kz workgroups per tile, and the sums
+ * go to kz partial rows in the scratch (same bits either way); *pend then describes the update still
+ * to apply (NkFoldArgs).
  * Returns 1 when no tile divides the output columns (the caller falls back), -2 when a fixed
  * scratch region is too small, else the launch status. */
 static int launch_mx_s(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid,
                        const mx_scratch_t *sc, nk_resid_t *pend) {
     const uint32_t kb = resid ? mx_kblocks(K) : 1;
-    const mx_tile_t *t = mx_pick(!a->A2, M, nout, K, glu, g_split == 0 ? 1 : kb);
+    uint32_t kz = 1;
+    const mx_tile_t *t = mx_pick(!a->A2, M, nout, K, glu, resid, kb, &kz);
     if (!t) return 1;
     const uint32_t tiles = mx_tiles(t, M, nout, glu);
-    uint32_t kz = 1;
     a->kblocks = 1;
     if (resid) {
         a->kblocks = kb;
-        /* split-row A: always (a block of 1024 is a workgroup's whole K loop elsewhere too; at 3584 rows
-         * FF down takes 63 us in four blocks against 67-79 unsplit, its four partial rows cost the
-         * LayerNorm that folds them 6 us more).  f32 A: below ~400 tiles */
-        if (kb > 1 && (g_split == 1 || (g_split < 0 && (a->A2 || tiles < 400)))) kz = kb;
         const size_t need = (size_t)kz * M * nout;
         if (sc && sc->ws) {
             /* a fixed region too small for the split may still hold the unsplit partial rows (same

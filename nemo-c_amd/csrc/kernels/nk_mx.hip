@@ -81,8 +81,8 @@ __device__ __forceinline__ void wait_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0
 
 /* PW: wavefronts that only load (0: the computing ones load).
  * EPI: 0 bias / activation / GLU / accumulate epilogue; 1 argmax keys; 2 blocked-K residual
- * update into partial rows.  AS: A as split rows; OS: outputs as split rows (EPI 0 without GLU). */
-template <int BM, int BN, int WGM, int WGN, int PW, int NS, bool GLU, int EPI, bool AS, bool OS>
+ * update into partial rows (TOT: the sum of several blocks stays in registers).  AS: A as split rows; OS: outputs as split rows (EPI 0 without GLU). */
+template <int BM, int BN, int WGM, int WGN, int PW, int NS, bool GLU, int EPI, bool AS, bool OS, bool TOT = false>
 __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const smem) {
     static_assert(!OS || (EPI == 0 && !GLU), "split outputs from the plain epilogue only");
     constexpr int NW = PW ? PW : WGM * WGN, KS = NK_MX_KS; /* NW: wavefronts that load */
@@ -219,26 +219,37 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
     /* lane l holds row 16 i + l % 16, columns 16 j + 4 (l / 16) + e of each tile */
     const u32 row0 = m0 + wm * WTM + fr;
     /* EPI 2, the residual update, deferred: the K blocks' sums go to partials[kz][row][n] (rows of N
-     * floats), (((0 + b0) + b1) + ...) where one workgroup computes several: the sum so far is read
-     * back from the partial row at each block's end instead of being kept in TI * TJ * 4 registers.
-     * The rows are folded into C in block order afterwards, by the LayerNorm that reads them next or
-     * by resid_fold: C + alpha * (((0 + p0) + p1) + ...), the unsplit epilogue's bits. */
-    auto add_block = [&](bool first) {
+     * floats), (((0 + b0) + b1) + ...) where one workgroup computes several.  The rows are folded
+     * into C in block order afterwards, by the LayerNorm that reads them next or by resid_fold:
+     * C + alpha * (((0 + p0) + p1) + ...), the unsplit epilogue's bits.  The sum so far is kept in
+     * registers (TOT: for kernels that run several blocks per workgroup) or read back from the
+     * partial row (kernels that run several only where the scratch holds no more parts). */
+    floatx4 tot[TOT ? TI : 1][TOT ? TJ : 1];
+    if constexpr (TOT)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) tot[i][j] = (floatx4){ 0.f, 0.f, 0.f, 0.f };
+    auto end_block = [&](bool first, bool last) {
         float *P = a.ws + (u64)kz * a.M * a.N + c0 + wn * WTN + 4 * fg;
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
-            if (row0 + 16 * i < M) {
-                floatx4 *p = (floatx4 *)(P + (u64)(row0 + 16 * i) * a.N);
-                floatx4 t[TJ];
+        for (int i = 0; i < TI; ++i) {
+            const bool in = row0 + 16 * i < M;
+            floatx4 *p = (floatx4 *)(P + (u64)(in ? row0 + 16 * i : M - 1) * a.N);
+            floatx4 t[TJ];
 #pragma unroll
-                for (int j = 0; j < TJ; ++j) t[j] = first ? (floatx4){ 0.f, 0.f, 0.f, 0.f } : p[4 * j];
-#pragma unroll
-                for (int j = 0; j < TJ; ++j) p[4 * j] = t[j] + acc[i][j];
+            for (int j = 0; j < TJ; ++j) {
+                if constexpr (TOT) t[j] = tot[i][j];
+                else t[j] = first ? (floatx4){ 0.f, 0.f, 0.f, 0.f } : p[4 * j];
             }
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) acc[i][j] = (floatx4){ 0.f, 0.f, 0.f, 0.f };
+            for (int j = 0; j < TJ; ++j) {
+                t[j] += acc[i][j];
+                if constexpr (TOT) tot[i][j] = t[j];
+                if (in && (!TOT || last)) p[4 * j] = t[j];
+                acc[i][j] = (floatx4){ 0.f, 0.f, 0.f, 0.f };
+            }
+        }
     };
     /* one 32-K substep: every hi product, then every lo product (the same order in every kernel, so
      * every tile gives the same bits).  The weights are the MFMA's first operand: a lane then holds
@@ -299,7 +310,7 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
         if (whole) mma(F[1]);
         if constexpr (EPI == 2) {
             if ((q + 1) % spb == 0) { /* a K block ends: add its sum, start the next from zero */
-                add_block(q + 1 == spb);
+                end_block(q + 1 == spb, q + 1 == nst);
             }
         }
     }
@@ -434,6 +445,12 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
     GEMM_MX(gemm_mx##T##_s_so, BM, BN, WGM, WGN, PW, NS, false, 0, true, true)                            \
     GEMM_MX(gemm_mx##T##_acc_s, BM, BN, WGM, WGN, PW, NS, false, 2, true, false)
 #define GEMM_MX_SG(T, BM, BN, WGM, WGN, PW, NS) GEMM_MX(gemm_mx##T##_glu_s, BM, BN, WGM, WGN, PW, NS, true, 0, true, false)
+/* a residual update whose workgroups run all K blocks */
+#define GEMM_MX_U(T, BM, BN, WGM, WGN, PW, NS)                                                            \
+    extern "C" __global__ __launch_bounds__(64 * (WGM * WGN + PW)) void gemm_mx##T##_acc_s(const NkGemmArgs a) { \
+        __shared__ uint4 ring_mem[NS * (BM * 2 + BN) * 8];                                                \
+        mx_impl<BM, BN, WGM, WGN, PW, NS, false, 2, true, false, true>(a, (lds_char_t *)ring_mem);        \
+    }
 /* and of f32 A */
 #define GEMM_MX_F(T, BM, BN, WGM, WGN, PW, NS)                                                            \
     GEMM_MX(gemm_mx##T, BM, BN, WGM, WGN, PW, NS, false, 0, false, false)                                 \
@@ -449,6 +466,7 @@ GEMM_MX_SG(64x128d, 64, 128, 2, 2, 4, 4)
 GEMM_MX_SS(64x64, 64, 64, 2, 2, 4, 3)
 GEMM_MX_SS(32x64, 32, 64, 2, 2, 4, 9)
 GEMM_MX_S(32x32, 32, 32, 2, 2, 4, 12)
+GEMM_MX_U(64x128u, 64, 128, 2, 2, 0, 2)
 GEMM_MX_FF(64x128, 64, 128, 2, 2, 4, 2)
 GEMM_MX_FF(64x64, 64, 64, 2, 2, 4, 3)
 GEMM_MX_FF(32x64, 32, 64, 2, 2, 4, 9)
