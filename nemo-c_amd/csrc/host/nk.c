@@ -781,6 +781,13 @@ int nk_conv2d_c1_s2_relu_b(gpu_t *g, const float *X, const float *W, const float
 
 int nk_dwconv2d_s2_b(gpu_t *g, const float *X, const float *W, const float *bias, float *Y, uint32_t T, uint32_t F,
                      uint32_t T1, uint32_t F1, uint32_t C, uint32_t batch) {
+    /* four channels and four outputs per thread from 256 positions on (64 windows of 19 x 33: 32.1 ->
+     * 13.3 us; 170 positions 4.0 us with one output per workgroup, 4.3 so) */
+    if ((uint64_t)T1 * F1 * batch >= 256 && T && F && C % 4 == 0 && C && C <= 1024 && 256 % (C / 4) == 0 && aligned16(X) && aligned16(Y) && aligned16(W) && aligned16(bias)) {
+        NkConvArgs v = { X, W, bias, Y, T, F, T1, F1, C, 0, T * F * C, T1 * F1 * C };
+        const uint32_t segs = T1 * ((F1 + 3) / 4), per = 256 / (C / 4);
+        return gpu_launch(g, "dwconv2d_s2_v4", &v, sizeof v, (segs + per - 1) / per, batch, 1, 256, 1, 1);
+    }
     const uint32_t fb = conv_fb(T1, F1, batch);
     NkConvArgs a = { X, W, bias, Y, T, F, T1, F1, C, fb, T * F * C, T1 * F1 * C };
     return gpu_launch(g, "dwconv2d_s2", &a, sizeof a, T1 * ((F1 + fb - 1) / fb), batch, 1, 256, 1, 1);
@@ -791,11 +798,12 @@ int nk_conv2d_c1_dw_s2_b(gpu_t *g, const float *X, const float *W0, const float 
                          uint32_t F2, uint32_t C, uint32_t batch) {
     if (F > NK_CONV02_FMAX) return gpu_fail(g, "nk_conv2d_c1_dw_s2: more than 256 mel bins");
     if (!T2 || !F2 || !batch) return 0;
-    /* whole output rows per workgroup when there are enough rows to fill the GPU; one column per
-     * workgroup for a single stream's few rows (measured: 8.6 us against 16.3 us with 4 columns
-     * for a 24-row window, 112 us with whole rows for 64 windows of 65 rows) */
+    /* output columns per workgroup: a workgroup's first output costs one more conv 0 column and its
+     * taps, a launch of few rows needs workgroups for every CU (of 33 columns, the best per row count: 7
+     * rows 1 column 3.8 us, 4.3 with 3; 19 rows 3, 4.4 us, 5.1 with 6; 76 rows 6, 6.3 / 7.2 with 11; 304
+     * rows 11, 12.4 / 13.3 with 17; 1216 rows 17, 30.6 / 31.8 with 11; 4864 rows all within 1%) */
     const uint64_t rows = (uint64_t)T2 * batch;
-    const uint32_t fb = rows >= 1024 ? F2 : rows >= 256 ? 4 : 1;
+    const uint32_t fb = rows < 16 ? 1 : rows < 64 ? 3 : rows < 256 ? 6 : rows < 1024 ? 11 : rows < 4096 ? 17 : F2;
     NkConv02Args a = { X, W0, b0, W2, b2, Y, T, F, T1, F1, T2, F2, C, fb, T * F, T2 * F2 * C };
     return gpu_launch(g, "conv2d_c1_dw_s2", &a, sizeof a, T2 * ((F2 + fb - 1) / fb), batch, 1, 256, 1, 1);
 }
@@ -810,6 +818,10 @@ int nk_mel_frames(gpu_t *g, const float *span, const int *tab, uint32_t F, const
 
 int nk_flatten_cf_b(gpu_t *g, const float *X, float *Y, uint32_t T, uint32_t F, uint32_t C, uint32_t batch) {
     NkFlatArgs a = { X, Y, T, F, C, 0 };
+    /* through LDS from half a million elements on (64 windows of 10 x 17 x 256: 9.9 -> 6.6 us; one window
+     * 2.8 us element by element, 3.6 so) */
+    if ((uint64_t)T * F * C * batch >= 500000 && C % 4 == 0 && (uint64_t)F * (C + 4) <= NK_FLAT_LDS && aligned16(X) && aligned16(Y) && T && batch)
+        return gpu_launch(g, "flatten_cf_t", &a, sizeof a, T, batch, 1, 256, 1, 1);
     return gpu_launch(g, "flatten_cf", &a, sizeof a, blocks_for((uint64_t)T * F * C), batch, 1, 256, 1, 1);
 }
 

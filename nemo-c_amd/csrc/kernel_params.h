@@ -37,6 +37,7 @@ typedef uint16_t u16;
 #define NK_LN_THREADS 256
 #define NK_ROW_MAX 4096         /* row width limit of the per-row kernels (4 float4 per thread)    */
 #define NK_CONV_TAPS 9          /* causal depthwise conv kernel size                               */
+#define NK_FLAT_LDS 5120        /* floats of LDS of the flatten kernel                             */
 #define NK_DW_ROWS 7            /* rows per workgroup of the batched depthwise conv (many rows)    */
 #define NK_FR_MAX_KC 1024       /* few-row MFMA GEMM: K columns of A staged per workgroup          */
 

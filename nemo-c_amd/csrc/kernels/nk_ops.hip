@@ -68,82 +68,131 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2(NkConvArgs a) {
     }
 }
 
+/* The same, four channels per thread (C / 4 divides 256, 16-byte aligned rows): a thread computes DW2_FB
+ * neighbouring outputs of one row, whose 9 input columns x 3 rows it loads at once (two new columns
+ * per output instead of three, one memory round trip per thread; the taps come through LDS, where a
+ * thread's 36 are nine 16-byte reads).  Positions outside X are products with zero.
+ * 64 windows of 19 x 33 x 256: 32.1 -> 13.3 us (52 MB read and written: 10.7 at the rate of a copy),
+ * 256 windows 120 -> 44 us. */
+#define DW2_FB 4
+extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
+    __shared__ floatx4 taps[1024 * 9 / 4];
+    const u32 C4 = a.C / 4, tid = threadIdx.x, per = 256 / C4;
+    const u32 nfb = (a.F1 + DW2_FB - 1) / DW2_FB, seg = blockIdx.x * per + tid / C4;
+    const u32 t1 = seg / nfb, f0 = (seg % nfb) * DW2_FB, c = 4 * (tid % C4);
+    const float *X = a.X + (u64)blockIdx.y * a.xs + c;
+    for (u32 i = tid; i < a.C * 9 / 4; i += 256) taps[i] = ((const floatx4 *)a.W)[i];
+    const bool in = t1 < a.T1;
+    floatx4 x[3][2 * DW2_FB + 1];
+#pragma unroll
+    for (int kh = 0; kh < 3; ++kh) {
+        const int ti = (int)(2 * t1 + kh) - 2;
+        const bool row = in && ti >= 0 && ti < (int)a.T;
+#pragma unroll
+        for (int k = 0; k < 2 * DW2_FB + 1; ++k) {
+            const int fi = (int)(2 * f0 + k) - 2;
+            const bool ok = row && fi >= 0 && fi < (int)a.F;
+            const floatx4 v = *(const floatx4 *)(X + (ok ? ((u64)ti * a.F + fi) * a.C : 0));
+            x[kh][k] = ok ? v : (floatx4){ 0.f, 0.f, 0.f, 0.f };
+        }
+    }
+    const floatx4 bias = *(const floatx4 *)(a.bias + c);
+    __syncthreads();
+    if (!in) return;
+    floatx4 w[9]; /* channel e, tap k is element 9 e + k */
+#pragma unroll
+    for (int k = 0; k < 9; ++k) w[k] = taps[(c / 4) * 9 + k];
+    float *Y = a.Y + (u64)blockIdx.y * a.ys + ((u64)t1 * a.F1 + f0) * a.C + c;
+#pragma unroll
+    for (int f = 0; f < DW2_FB; ++f) {
+        if (f0 + f >= a.F1) break;
+        floatx4 acc = bias;
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += w[(9 * e + k) / 4][(9 * e + k) % 4] * x[k / 3][2 * f + k % 3][e];
+        *(floatx4 *)(Y + (u64)f * a.C) = acc;
+    }
+}
+
 /* conv 0 (1 -> C channels + ReLU) followed by conv 2 (depthwise, + bias) without storing conv 0's
  * output: X [T][F] -> Y [T2][F2][C].  Workgroup = one output row t2 and fb output columns of one
  * window; thread = channel.  The seven X rows the output row reads (4 t2 - 6 .. 4 t2) are staged
  * in LDS.  Every conv 0 value is computed exactly as conv2d_c1_s2_relu computes it (bias, then the
  * taps in (kh, kw) order, taps outside X skipped, ReLU) and every output exactly as dwconv2d_s2
  * computes it (bias, then the taps in order, positions outside conv 0's T1 x F1 skipped), so the
- * result equals the two kernels' bit for bit.  A thread walks its columns left to right; for each
- * it reads the 7 x 7 mel values its conv 0 taps can touch (columns 4 f2 - 6 .. 4 f2) from LDS
- * into registers once (a third fewer LDS reads than per tap: 8.6 -> 5.7 us for one 24-row window,
- * 564 -> 386 us for 256 windows of 121 rows), and the conv 0 column 2 f2 of output f2, which is
- * column 2 (f2 + 1) - 2 of the next, is kept. */
+ * result equals the two kernels' bit for bit (finite weights: a skipped tap is added here as a
+ * product with zero).
+ *
+ * Bound by its 63 multiply-adds per output (17 us for 64 windows of 72 rows at the full vector rate), so
+ * everything else is kept out of the loop: the mel rows lie in LDS with zeros around them, so no tap
+ * is tested; a thread walks its columns left to right and reads the four new mel columns of each
+ * output as one 16-byte broadcast per row (seven LDS reads where every column was read by itself, 49),
+ * and the conv 0 column 2 f2 of output f2, which is column 2 (f2 + 1) - 2 of the next, is kept.
+ * Positions outside conv 0 are masked, not branched around.  One window of 72 rows 8.4 -> 4.4 us, 64
+ * windows 73 -> 30.6, 256 windows 216 -> 103. */
+#define CONV02_PAD 7 /* LDS index of mel column 0: the four new columns of output f2 start at 4 f2 + 4 */
 extern "C" __global__ __launch_bounds__(256) void conv2d_c1_dw_s2(NkConv02Args a) {
-    __shared__ float xs[7][NK_CONV02_FMAX];
+    constexpr u32 LDW = NK_CONV02_FMAX + 16;
+    __shared__ __attribute__((aligned(16))) float xs[7][LDW];
     const u32 nfb = (a.F2 + a.fb - 1) / a.fb;
     const u32 t2 = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * a.fb;
     const float *X = a.X + (u64)blockIdx.y * a.xs;
     float *Y = a.Y + (u64)blockIdx.y * a.ys;
     const u32 fe = min(f0 + a.fb, a.F2);
     const int ti0 = 4 * (int)t2 - 6; /* X row of LDS row 0 */
-    for (u32 i = threadIdx.x; i < 7 * a.F; i += 256) {
-        const int r = (int)(i / a.F), ti = ti0 + r;
-        xs[r][i % a.F] = (ti >= 0 && ti < (int)a.T) ? X[(u64)ti * a.F + i % a.F] : 0.0f;
+    /* the LDS columns this workgroup's outputs read */
+    const u32 i0 = min(4 * f0, LDW - 4), iw = min(4 * fe + 4, LDW) - i0;
+    for (u32 i = threadIdx.x; i < 7 * iw; i += 256) {
+        const u32 r = i / iw, k = i0 + i % iw;
+        const int ti = ti0 + (int)r, col = (int)k - CONV02_PAD;
+        xs[r][k] = ti >= 0 && ti < (int)a.T && col >= 0 && col < (int)a.F ? X[(u64)ti * a.F + col] : 0.0f;
     }
     __syncthreads();
+    u32 row_in[3]; /* all ones for the conv 0 rows 2 t2 - 2 .. 2 t2 that exist */
+#pragma unroll
+    for (int k = 0; k < 3; ++k) row_in[k] = (u32)(2 * (int)t2 + k - 2) < a.T1 ? ~0u : 0u;
     for (u32 c = threadIdx.x; c < a.C; c += 256) {
         float w0[9], w2[9];
 #pragma unroll
         for (int k = 0; k < 9; ++k) { w0[k] = a.W0[c * 9 + k]; w2[k] = a.W2[c * 9 + k]; }
         const float bias0 = a.b0[c], bias2 = a.b2[c];
-        float keep[3];
-        bool keep_ok[3];
+        /* mel columns 4 f2 - 6 .. 4 f2 of the seven rows; conv 0's column 2 f2 - 2 of output f2 */
+        float xv[7][7], keep[3];
+        /* conv 0 at row 2 t2 + kh2 - 2, column f1: mel row 2 kh2 + kh, columns q .. q + 2 of xv */
+        auto conv0 = [&](const int kh2, const int q, const u32 f1) -> float {
+            float acc = bias0;
+#pragma unroll
+            for (int kh = 0; kh < 3; ++kh)
+#pragma unroll
+                for (int kw = 0; kw < 3; ++kw) acc += w0[kh * 3 + kw] * xv[2 * kh2 + kh][q + kw];
+            const u32 in = row_in[kh2] & (f1 < a.F1 ? ~0u : 0u); /* uniform: a mask, not a branch */
+            return __uint_as_float(__float_as_uint(fmaxf(acc, 0.0f)) & in);
+        };
+#pragma unroll
+        for (int r = 0; r < 7; ++r)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) xv[r][4 + q] = xs[r][min(4 * f0 + 1 + q, LDW - 1)];
+#pragma unroll
+        for (int kh2 = 0; kh2 < 3; ++kh2) keep[kh2] = conv0(kh2, 4, 2 * f0 - 2);
         for (u32 f2 = f0; f2 < fe; ++f2) {
-            /* mel columns 4 f2 - 6 .. 4 f2 of the 7 rows (reads clamped into the row; taps outside
-             * the mel window are skipped below, as in conv2d_c1_s2_relu) */
-            float xv[7][7];
-            const int cb = 4 * (int)f2 - 6;
 #pragma unroll
-            for (int r = 0; r < 7; ++r)
+            for (int r = 0; r < 7; ++r) {
+                const floatx4 n = *(const floatx4 *)&xs[r][min(4 * f2 + 4, LDW - 4)];
 #pragma unroll
-                for (int q = 0; q < 7; ++q) xv[r][q] = xs[r][min(max(cb + q, 0), (int)a.F - 1)];
-            /* conv 0 at row 2 t2 + kh2 - 2, column 2 f2 - 2 + cs: mel row 2 kh2 + kh of xv, column 2 cs + kw */
-            auto conv0 = [&](const int kh2, const int cs, bool &ok) -> float {
-                const int t1 = 2 * (int)t2 + kh2 - 2, f1 = 2 * (int)f2 - 2 + cs;
-                ok = t1 >= 0 && t1 < (int)a.T1 && f1 >= 0 && f1 < (int)a.F1;
-                if (!ok) return 0.0f;
-                float acc = bias0;
+                for (int q = 0; q < 3; ++q) xv[r][q] = xv[r][4 + q];
 #pragma unroll
-                for (int kh = 0; kh < 3; ++kh) {
-                    const int ti = 2 * t1 + kh - 2;
-                    if (ti < 0 || ti >= (int)a.T) continue;
-#pragma unroll
-                    for (int kw = 0; kw < 3; ++kw) {
-                        const int fi = 2 * f1 + kw - 2;
-                        if (fi < 0 || fi >= (int)a.F) continue;
-                        acc += w0[kh * 3 + kw] * xv[2 * kh2 + kh][2 * cs + kw];
-                    }
-                }
-                return fmaxf(acc, 0.0f);
-            };
-            float v[3][3];
-            bool ok[3][3];
-#pragma unroll
-            for (int kh2 = 0; kh2 < 3; ++kh2) {
-                if (f2 == f0) v[kh2][0] = conv0(kh2, 0, ok[kh2][0]);
-                else { v[kh2][0] = keep[kh2]; ok[kh2][0] = keep_ok[kh2]; }
-                v[kh2][1] = conv0(kh2, 1, ok[kh2][1]);
-                v[kh2][2] = conv0(kh2, 2, ok[kh2][2]);
-                keep[kh2] = v[kh2][2];
-                keep_ok[kh2] = ok[kh2][2];
+                for (int q = 0; q < 4; ++q) xv[r][3 + q] = n[q];
             }
             float acc = bias2;
 #pragma unroll
-            for (int kh2 = 0; kh2 < 3; ++kh2)
-#pragma unroll
-                for (int kw2 = 0; kw2 < 3; ++kw2)
-                    if (ok[kh2][kw2]) acc += w2[kh2 * 3 + kw2] * v[kh2][kw2];
+            for (int kh2 = 0; kh2 < 3; ++kh2) {
+                const float v1 = conv0(kh2, 2, 2 * f2 - 1), v2 = conv0(kh2, 4, 2 * f2);
+                acc += w2[kh2 * 3] * keep[kh2];
+                acc += w2[kh2 * 3 + 1] * v1;
+                acc += w2[kh2 * 3 + 2] * v2;
+                keep[kh2] = v2;
+            }
             Y[((u64)t2 * a.F2 + f2) * a.C + c] = acc;
         }
     }
@@ -191,6 +240,29 @@ extern "C" __global__ __launch_bounds__(256) void mel_frames(const NkMelArgs a) 
 
 /* [T][F][C] -> [T][C*F] channel-major flatten: reference src/kernels.metal:456-462.
  * One thread per output element (reads gather, writes are coalesced). */
+/* one [F][C] row of a window per workgroup through LDS (F (C + 4) floats of at most NK_FLAT_LDS, C % 4
+ * == 0, 16-byte aligned), so that both the reads and the writes are whole lines; a thread's own
+ * elements were C apart.  LDS rows are C + 4 floats, which spreads the reads along f over the banks.
+ * 64 windows of 10 x 17 x 256: 9.9 -> 6.6 us, 256 windows 30.1 -> 16.2. */
+extern "C" __global__ __launch_bounds__(256) void flatten_cf_t(const NkFlatArgs a) {
+    __shared__ __attribute__((aligned(16))) float s[NK_FLAT_LDS];
+    const u64 base = ((u64)blockIdx.y * a.T + blockIdx.x) * a.F * a.C;
+    const u32 n4 = a.F * a.C / 4, C4 = a.C / 4;
+    for (u32 i = threadIdx.x; i < n4; i += 256)
+        *(floatx4 *)&s[(i / C4) * (a.C + 4) + 4 * (i % C4)] = *(const floatx4 *)(a.X + base + 4 * (u64)i);
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < n4; i += 256) {
+        u32 c = 4 * i / a.F, f = 4 * i - c * a.F;
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = s[f * (a.C + 4) + c];
+            if (++f == a.F) { f = 0; ++c; }
+        }
+        *(floatx4 *)(a.Y + base + 4 * (u64)i) = v;
+    }
+}
+
 extern "C" __global__ __launch_bounds__(256) void flatten_cf(NkFlatArgs a) {
     const u64 idx = (u64)blockIdx.x * 256 + threadIdx.x;
     const u64 total = (u64)a.T * a.C * a.F;

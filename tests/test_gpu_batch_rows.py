@@ -90,3 +90,46 @@ def test_dwconv_runs(gpu, D, order):
     pick = list(range(90)) + [M - 1]
     ref = np.concatenate([oracle.dwconv_ln_silu(din[table[i][0] - 8:table[i][0] + 1], W, g, b, 1) for i in pick])
     assert rel_err(y[pick], ref) < 1e-5
+
+
+@pytest.mark.parametrize("T,F,C,batch", [(19, 33, 256, 9), (20, 30, 256, 7), (37, 65, 32, 5), (33, 31, 1024, 2), (64, 9, 4, 40)])
+def test_dwconv2d_forms(gpu, T, F, C, batch):
+    """The four-channel form against the one-channel form (taken for rows off 16 bytes), bit for bit, on
+    even and odd sizes, a last group of fewer than four outputs and several segments per workgroup."""
+    import nemoasr
+
+    L = nemoasr.lib()
+    rng = np.random.default_rng([T, F, C])
+    T1, F1 = T // 2 + 1, F // 2 + 1
+    assert T1 * F1 * batch >= 256
+    X = rng.standard_normal((batch, T, F, C)).astype(np.float32)
+    W, b = (rng.standard_normal((C, 9)) / 3).astype(np.float32), rng.standard_normal(C).astype(np.float32)
+    dX, dW, db = gpu.put(X), gpu.put(W), gpu.put(b)
+    off = gpu.alloc(X.nbytes + 4)
+    off.write(X, 4)
+    dY, dZ = (gpu.alloc(batch * T1 * F1 * C * 4) for _ in range(2))
+    gpu.begin()
+    gpu.check(L.nk_dwconv2d_s2_b(gpu.h, dX.ptr, dW.ptr, db.ptr, dY.ptr, T, F, T1, F1, C, batch))
+    gpu.check(L.nk_dwconv2d_s2_b(gpu.h, off.at(4), dW.ptr, db.ptr, dZ.ptr, T, F, T1, F1, C, batch))
+    gpu.end()
+    y = dY.read((batch, T1, F1, C))
+    assert np.array_equal(bits(y), bits(dZ.read(y.shape)))
+    assert rel_err(y[-1], oracle.dwconv2d_s2(X[-1], W, b)) < 1e-6
+
+
+@pytest.mark.parametrize("T,F,C,batch", [(10, 17, 256, 12), (3, 5, 1016, 33), (9, 11, 36, 141)])
+def test_flatten_forms(gpu, T, F, C, batch):
+    """Through LDS (half a million elements or more) and element by element: the transpose itself."""
+    import nemoasr
+
+    L = nemoasr.lib()
+    assert T * F * C * batch >= 500000
+    X = np.random.default_rng(T).standard_normal((batch, T, F, C)).astype(np.float32)
+    dX, dY, dZ = gpu.put(X), gpu.alloc(X.nbytes), gpu.alloc(X[0].nbytes)
+    gpu.begin()
+    gpu.check(L.nk_flatten_cf_b(gpu.h, dX.ptr, dY.ptr, T, F, C, batch))
+    gpu.check(L.nk_flatten_cf_b(gpu.h, dX.ptr, dZ.ptr, T, F, C, 1))
+    gpu.end()
+    ref = np.ascontiguousarray(X.transpose(0, 1, 3, 2)).reshape(batch, T, C * F)
+    assert np.array_equal(dY.read(ref.shape), ref)
+    assert np.array_equal(dZ.read(ref[0].shape), ref[0])
