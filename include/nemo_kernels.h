@@ -100,8 +100,8 @@ int nk_gemm_argmax_rows(gpu_t *g, const float *A, uint32_t lda, const uint16_t *
 int nk_gemm_ksplit(int mode);
 /* Many-row tile: -1 (default) by an estimate of the time from the shape, else 0 128x256 (split-row A),
  * 1 64x128, 2 64x64, 3 32x64, 4 32x32, 5 64x128 with a deeper ring (split-row A), 6 64x128 with the
- * K blocks' sum in registers (split-row residual updates) where the tile exists and divides the output
- * columns.  All give the same bits.  Returns the previous setting. */
+ * K blocks' sum in registers (split-row residual updates), 7 96x256 (split-row A) where the tile exists
+ * and divides the output columns.  All give the same bits.  Returns the previous setting. */
 int nk_gemm_mx_tile(int t);
 /* Few-row residual updates (5..16 rows): 1 (default) splits K over four workgroups whose partial
  * rows are added in split order by a second launch, 0 keeps K in one workgroup (more wavefronts).

@@ -13,7 +13,7 @@ static int g_mx_tile = -1; /* many-row tile: -1 by estimate, else an index of mx
 
 int nk_gemm_mx_tile(int t) {
     const int prev = g_mx_tile;
-    g_mx_tile = t < 0 || t > 6 ? -1 : t;
+    g_mx_tile = t < 0 || t > 7 ? -1 : t;
     return prev;
 }
 
@@ -161,13 +161,14 @@ typedef struct {
     struct { float fix, step, fix1, step1; } us[2]; /* fix 0: not built for this form */
 } mx_tile_t;
 static const mx_tile_t mx_tile[] = { /* in the order of nk_gemm_mx_tile's numbers */
-    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.70f, 5.0f, 1.50f }, { 0 } } },
+    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.70f, 5.0f, 1.65f }, { 0 } } },
     { "64x128", 64, 128, 512, 512, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
     { "64x64", 64, 64, 512, 512, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
     { "32x64", 32, 64, 256, 512, 512, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
     { "32x32", 32, 32, 256, 512, 512, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
     { "64x128d", 64, 128, 256, 768, 512, { { 3.0f, 0.58f, 2.2f, 0.57f }, { 0 } } },
     { "64x128u", 64, 128, 512, 256, 0, { { 3.5f, 0.95f, 3.0f, 0.76f }, { 0 } } }, /* residual updates, K not split */
+    { "96x256", 96, 256, 256, 512, 512, { { 4.0f, 1.40f, 4.0f, 1.40f }, { 0 } } },
 };
 #define MX_TILES ((int)(sizeof mx_tile / sizeof *mx_tile))
 

@@ -19,8 +19,8 @@
  * and then waits for its fragment reads.
  *   - PW = 4: four more wavefronts only load, so the computing ones never issue a DMA; 18 rows,
  *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 13.4, FF down 13.8 -> 12.1.  All tiles but one.
- *   - PW = 0: 128x256 computed and loaded by eight wavefronts (two per SIMD, 198 VGPRs each: no room
- *     for loaders), half the staged bytes per MFMA of 64x128: its steps of 1.5 us run at 1.2 PFLOP/s
+ *   - PW = 0: 128x256 and 96x256 computed and loaded by eight wavefronts (two per SIMD, 198 VGPRs
+ *     each: no room for loaders; 192x256 spills), half the staged bytes per MFMA of 64x128: its steps of 1.5 us run at 1.2 PFLOP/s
  *     issued, the rate of a large library product here; 3584 rows, FF up 81.7 -> 68.6 us, pw1
  *     40.4 -> 29.0 us.
  * In both, a step's fragments are in registers one 32-K substep ahead of their MFMAs, so LDS latency
@@ -423,7 +423,9 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
     }
 }
 
-/* Tiles and ring depths.  64x128 and 64x64 fit two workgroups on a CU (2 x 64 KB, 2 x 72 KB of its
+/* Tiles and ring depths.  128x256 and 96x256 take a CU each; which of the two leaves fewer CUs idle
+ * depends on the rows (1300 rows, FF up in one round of 224 tiles of 96x256 29.9 us, 176 of 128x256 34.9; 3584
+ * rows, QKV 49.1 against 57.1, FF up 77.3 against 69.6).  64x128 and 64x64 fit two workgroups on a CU (2 x 64 KB, 2 x 72 KB of its
  * 160 KB of LDS): one's MFMAs run while the other waits at its barrier, the better choice once there
  * are more than 256 workgroups.  64x128d (four stages), 32x64 and 32x32 take a CU each, with nearly
  * all of a 1024-column K loop's loads in flight at once: for launches of up to 256 workgroups, whose
@@ -460,6 +462,7 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
 #define GEMM_MX_SS(...) GEMM_MX_S(__VA_ARGS__) GEMM_MX_SG(__VA_ARGS__)
 #define GEMM_MX_FF(...) GEMM_MX_F(__VA_ARGS__) GEMM_MX_FG(__VA_ARGS__)
 GEMM_MX_SS(128x256, 128, 256, 2, 4, 0, 2)
+GEMM_MX_SS(96x256, 96, 256, 2, 4, 0, 2)
 GEMM_MX_SS(64x128, 64, 128, 2, 2, 4, 2)
 GEMM_MX_S(64x128d, 64, 128, 2, 4, 4, 4)
 GEMM_MX_SG(64x128d, 64, 128, 2, 2, 4, 4)

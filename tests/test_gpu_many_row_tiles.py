@@ -16,7 +16,7 @@ from test_gpu_split import bits, split_rows, w_bf16
 
 pytestmark = pytest.mark.gpu
 
-TILES = [0, 1, 2, 3, 4, 5, 6, -1]
+TILES = [0, 1, 2, 3, 4, 5, 6, 7, -1]
 
 
 def reference(A, W, bias, act, split):
@@ -38,7 +38,7 @@ def reference(A, W, bias, act, split):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 256, 64), (32, 256, 128), (33, 512, 704), (64, 256, 1024), (65, 1024, 192),
-                                   (129, 512, 1024), (300, 2048, 256), (18, 256, 96), (65, 256, 32), (70, 512, 1056),
+                                   (97, 512, 320), (129, 512, 1024), (300, 2048, 256), (18, 256, 96), (65, 256, 32), (70, 512, 1056),
                                    (50, 256, 2048)])
 @pytest.mark.parametrize("form", ["plain", "bias_relu", "silu_split", "glu_rows", "odd_ldc", "resid"])
 def test_tiles_agree(gpu, M, N, K, form):
