@@ -18,11 +18,11 @@
  * instruction (four wavefronts on a CU stream 138 GB/s, eight 217, sixteen 323, measured from L2)
  * and then waits for its fragment reads.
  *   - PW = 4: four more wavefronts only load, so the computing ones never issue a DMA; 18 rows,
- *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 13.4, FF down 13.8 -> 12.1.  All tiles but one.
+ *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 13.4, FF down 13.8 -> 12.1.  All tiles but two.
  *   - PW = 0: 128x256 and 96x256 computed and loaded by eight wavefronts (two per SIMD, 198 VGPRs
- *     each: no room for loaders; 192x256 spills), half the staged bytes per MFMA of 64x128: its steps of 1.5 us run at 1.2 PFLOP/s
- *     issued, the rate of a large library product here; 3584 rows, FF up 81.7 -> 68.6 us, pw1
- *     40.4 -> 29.0 us.
+ *     each: no room for loaders; 192x256 spills), half the staged bytes per MFMA of 64x128: the steps of
+ *     128x256 take 1.5 us, 1.2 PFLOP/s issued, the rate of a large library product here; 3584
+ *     rows, FF up 81.7 -> 68 us, pw1 40.4 -> 29.0 us.
  * In both, a step's fragments are in registers one 32-K substep ahead of their MFMAs, so LDS latency
  * is covered by the other substep's MFMAs; the accumulators stay in VGPRs; the weights are the
  * MFMA's first operand, so a lane holds four consecutive output columns and stores 8 or 16 bytes at
