@@ -87,8 +87,10 @@ void gpu_graph_free(gpu_graph_t *gr);
 int gpu_capturing(const gpu_t *g);
 
 /* Scratch of the split-K partial rows (GPU_SCRATCH_FLOATS allocated at creation): a larger request
- * grows it outside a capture and returns NULL (no error recorded) inside one.  Launches on one
- * gpu_t run in stream order, so they share it; it holds one pending residual update at a time. */
+ * grows it outside a capture and returns NULL (no error recorded) inside one.  A block whose address
+ * a capture took stays allocated until gpu_destroy, so graphs captured before the growth may be
+ * replayed after it.  Launches on one gpu_t run in stream order, so they share it; it holds one
+ * pending residual update at a time. */
 #define GPU_SCRATCH_FLOATS (1u << 20)
 float *gpu_scratch_ws(gpu_t *g, size_t floats_needed);
 

@@ -20,6 +20,7 @@ extern const unsigned char nk_code_object_end[];
 
 #define GPU_MAX_FN 96
 #define GPU_MAX_TIMED 32768
+#define GPU_MAX_RETIRED 40 /* scratch blocks that graphs hold: each at least twice the one before */
 
 struct gpu {
     int dev;
@@ -37,6 +38,9 @@ struct gpu {
     int nfn;
     float *ws;
     size_t ws_floats;
+    int ws_captured;                 /* a capture recorded the address of ws */
+    float *retired[GPU_MAX_RETIRED]; /* outgrown scratch that captured graphs still write */
+    int nretired;
     uint64_t launches;
     /* constant tables for kernels that take no optional pointers: rows 0..GPU_IOTA_N-1 and zeros */
     int *iota;
@@ -156,6 +160,7 @@ void gpu_destroy(gpu_t *g) {
         free(g->tbytes);
     }
     if (g->ws) hipFree(g->ws);
+    for (int i = 0; i < g->nretired; ++i) hipFree(g->retired[i]);
     if (g->iota) hipFree(g->iota);
     if (g->zeros) hipFree(g->zeros);
     hipEventDestroy(g->ev0);
@@ -538,16 +543,24 @@ void gpu_graph_free(gpu_graph_t *gr) {
     free(gr);
 }
 
+/* A graph keeps the address it was captured with, so a block that a capture was given is not freed
+ * when it is outgrown but kept until the context goes.  Its successor has at least twice its size (as
+ * long as that much memory is free), so the kept blocks together are smaller than the current one. */
 float *gpu_scratch_ws(gpu_t *g, size_t floats) {
     if (floats > g->ws_floats) {
-        if (g->capturing) return NULL;
+        if (g->capturing || (g->ws_captured && g->nretired == GPU_MAX_RETIRED)) return NULL;
+        const size_t twice = g->ws_captured && floats < 2 * g->ws_floats ? 2 * g->ws_floats : floats;
         hipStreamSynchronize(g->stream);
         float *p = NULL;
-        if (hipMalloc((void **)&p, floats * sizeof(float)) != hipSuccess) return NULL;
-        if (g->ws) hipFree(g->ws);
+        if (hipMalloc((void **)&p, twice * sizeof(float)) == hipSuccess) floats = twice;
+        else if (twice == floats || hipMalloc((void **)&p, floats * sizeof(float)) != hipSuccess) return NULL;
+        if (g->ws_captured) g->retired[g->nretired++] = g->ws;
+        else if (g->ws) hipFree(g->ws);
         g->ws = p;
         g->ws_floats = floats;
+        g->ws_captured = 0;
     }
+    if (g->capturing) g->ws_captured = 1;
     return g->ws;
 }
 
