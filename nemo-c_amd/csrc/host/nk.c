@@ -751,8 +751,9 @@ int nk_dwconv_ln_silu_rows_split(gpu_t *g, const float *din_base, const int *row
     /* seven rows per workgroup from 1200 rows on, where their workgroups fill the GPU (chunks of 14 or 7
      * rows, graph-replayed: 448 rows 7.9 us against 6.8 one row per workgroup, 1792 12.7 / 14.9, 3584
      * 16.9 / 25.6; chunks of 4: 2400 17.4 / 18.7; of 2: 4000 26.8 / 31.0; of 1: 2000 rows 22.7 / 18.6);
-     * 16-byte loads of the taps into LDS, four channels per thread */
-    if (M >= 1200 && D <= 4 * NK_LN_THREADS && aligned16(W))
+     * 16-byte loads of the taps into LDS, four channels per thread.  It reads the row table; without
+     * one (one run of rows from din_base on) the one-row kernel */
+    if (rows && M >= 1200 && D <= 4 * NK_LN_THREADS && aligned16(W))
         return gpu_launch(g, "dwconv_rows", &a, sizeof a, (M + NK_DW_ROWS - 1) / NK_DW_ROWS, 1, 1, NK_LN_THREADS, 1, 1);
     return gpu_launch(g, "dwconv_ln_silu", &a, sizeof a, M, 1, 1, NK_LN_THREADS, 1, 1);
 }

@@ -92,6 +92,25 @@ def test_dwconv_runs(gpu, D, order):
     assert rel_err(y[pick], ref) < 1e-5
 
 
+@pytest.mark.parametrize("M", [5, 1199, 1200, 3001])
+def test_dwconv_rows_without_table(gpu, M):
+    """No row table: the rows of one run from din_base on, as nk_dwconv_ln_silu, at every row count."""
+    import nemoasr
+
+    L = nemoasr.lib()
+    D = 64
+    rng = np.random.default_rng(M)
+    din, W = rng.standard_normal((M + 8, D)).astype(np.float32), (rng.standard_normal((D, 9)) / 3).astype(np.float32)
+    g, b = (1 + 0.1 * rng.standard_normal(D)).astype(np.float32), (0.1 * rng.standard_normal(D)).astype(np.float32)
+    ddin, dW, dg, db = (gpu.put(x) for x in (din, W, g, b))
+    dY, dZ = gpu.alloc(M * D * 4), gpu.alloc(M * D * 4)
+    gpu.begin()
+    gpu.check(L.nk_dwconv_ln_silu(gpu.h, ddin.ptr, dW.ptr, dg.ptr, db.ptr, dY.ptr, M, D, 9, 1e-5))
+    gpu.check(L.nk_dwconv_ln_silu_rows(gpu.h, ddin.ptr, None, M, dW.ptr, dg.ptr, db.ptr, dZ.ptr, D, 9, 1e-5))
+    gpu.end()
+    assert np.array_equal(bits(dZ.read((M, D))), bits(dY.read((M, D))))
+
+
 @pytest.mark.parametrize("T,F,C,batch", [(19, 33, 256, 9), (20, 30, 256, 7), (37, 65, 32, 5), (33, 31, 1024, 2), (64, 9, 4, 40)])
 def test_dwconv2d_forms(gpu, T, F, C, batch):
     """The four-channel form against the one-channel form (taken for rows off 16 bytes), bit for bit, on
