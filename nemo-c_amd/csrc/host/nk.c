@@ -748,13 +748,20 @@ int nk_dwconv_ln_silu_rows_split(gpu_t *g, const float *din_base, const int *row
     if (D > NK_ROW_MAX || D % 4 || taps != NK_CONV_TAPS) return bad(g, "dwconv: 9 taps, D a multiple of 4, at most 4096");
     if (!Y == !Ys || (uintptr_t)Ys % 8) return bad(g, "dwconv: one output form");
     NkDwArgs a = { din_base, W, gamma, beta, Y, NULL, rows, M, D, taps, eps, Ys };
-    /* seven rows per workgroup from 1200 rows on, where their workgroups fill the GPU (chunks of 14 or 7
-     * rows, graph-replayed: 448 rows 7.9 us against 6.8 one row per workgroup, 1792 12.7 / 14.9, 3584
-     * 16.9 / 25.6; chunks of 4: 2400 17.4 / 18.7; of 2: 4000 26.8 / 31.0; of 1: 2000 rows 22.7 / 18.6);
-     * 16-byte loads of the taps into LDS, four channels per thread.  It reads the row table; without
-     * one (one run of rows from din_base on) the one-row kernel */
-    if (rows && M >= 1200 && D <= 4 * NK_LN_THREADS && aligned16(W))
-        return gpu_launch(g, "dwconv_rows", &a, sizeof a, (M + NK_DW_ROWS - 1) / NK_DW_ROWS, 1, 1, NK_LN_THREADS, 1, 1);
+    /* from 1200 rows on several rows per workgroup: two, or seven from 3000 rows on, where their
+     * workgroups fill the GPU.  The lines are where they win, or lose at most 3%, at every chunk length
+     * (the host does not see the table), D 1024, graph-replayed, chunks of 1 / 2 / 4 / 7 / 14:
+     * 1200 rows, one row 11.8 / 11.8 / 11.7 / 11.7 / 11.5 us, two 12.1 / 9.7 / 9.6 / 10.1 / 9.5, seven 15.8 /
+     * 13.7 / 12.8 / 10.4 / 10.4; 2600 rows, one 24.3 / 20.2 / 20.2 / 20.1 / 19.9, two 20.9 / 14.8 / 14.8 /
+     * 15.3 / 14.8, seven 25.2 / 19.5 / 17.9 / 15.0 / 14.9; 3200 rows, one 30.5 / 23.5 / 23.5 / 23.6 / 23.2,
+     * two 24.4 / 17.3 / 17.3 / 17.6 / 17.2, seven 27.7 / 21.3 / 19.1 / 16.1 / 15.9.  16-byte loads of the
+     * taps into LDS, four channels per thread.  Both read the row table; without one (one run of rows
+     * from din_base on) the one-row kernel */
+    if (rows && M >= 1200 && D <= 4 * NK_LN_THREADS && aligned16(W)) {
+        const uint32_t R = M >= 3000 ? NK_DW_ROWS : NK_DW_ROWS_FEW;
+        return gpu_launch(g, R == NK_DW_ROWS ? "dwconv_rows" : "dwconv_rows_few", &a, sizeof a, (M + R - 1) / R, 1, 1,
+                          NK_LN_THREADS, 1, 1);
+    }
     return gpu_launch(g, "dwconv_ln_silu", &a, sizeof a, M, 1, 1, NK_LN_THREADS, 1, 1);
 }
 

@@ -39,6 +39,7 @@ typedef uint16_t u16;
 #define NK_CONV_TAPS 9          /* causal depthwise conv kernel size                               */
 #define NK_FLAT_LDS 5120        /* floats of LDS of the flatten kernel                             */
 #define NK_DW_ROWS 7            /* rows per workgroup of the batched depthwise conv (many rows)    */
+#define NK_DW_ROWS_FEW 2        /* and where those would be too few workgroups                     */
 #define NK_FR_MAX_KC 1024       /* few-row MFMA GEMM: K columns of A staged per workgroup          */
 
 enum { NK_ACT_NONE = 0, NK_ACT_SILU = 1, NK_ACT_RELU = 2, NK_ACT_GLU = 3 };

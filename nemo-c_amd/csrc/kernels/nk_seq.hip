@@ -555,11 +555,14 @@ extern "C" __global__ __launch_bounds__(256) void dwconv_ln_silu(const NkDwArgs 
  * through LDS by direct loads in whole lines, once for all rows, rows on consecutive cache rows (one
  * chunk's) read rows + 8 input rows instead of 9 each, and the two LayerNorm reductions of all rows
  * share two barriers.  Other tables (several chunks in one workgroup) load each row's nine input rows,
- * one row ahead of its sums; a row's sums are the same either way.  3584
- * rows (256 chunks of 14), graph-replayed: 25.6 -> 16.9 us, of which 7.6 are one workgroup's latency
- * and a launch (37 MB read and written: 7.6 us at the rate of a copy). */
-#define DWR NK_DW_ROWS
-extern "C" __global__ __launch_bounds__(256) void dwconv_rows(const NkDwArgs a) {
+ * one row ahead of its sums; a row's sums are the same either way.
+ * Seven rows divide the chunks of 7 and 14 and read the fewest input rows: 3584 rows (256 chunks of
+ * 14), graph-replayed, 25.5 -> 16.7 us, of which 7.6 are one workgroup's latency and a launch (37 MB
+ * read and written: 7.6 us at the rate of a copy).  With fewer than about 400 workgroups their rows
+ * one after another are the time, most of all where no two are of one chunk; two rows are loaded at
+ * once: 2000 rows of chunks of 1 / 2 / 4 / 14, one row per workgroup 19.6 / 16.5 / 16.5 / 16.2 us,
+ * two 16.7 / 12.2 / 12.2 / 12.2, seven 23.3 / 18.6 / 17.2 / 13.8. */
+template <int DWR> __device__ __forceinline__ void dwconv_rows_impl(const NkDwArgs &a) {
     __shared__ uint4 taps[(1024 * DW_TAPS * 4 + 1008) / 16];
     __shared__ float red[2][DWR][4];
     const u32 m = blockIdx.x * DWR, tid = threadIdx.x, lane = tid & 63, D4 = a.D >> 2;
@@ -620,7 +623,7 @@ extern "C" __global__ __launch_bounds__(256) void dwconv_rows(const NkDwArgs a) 
             if (r + 2 < DWR) load(r + 2, r & 1);
         }
     }
-    /* LayerNorm of the rows (those past n repeat row n - 1), dwconv_ln_silu's sums in its order */
+    /* LayerNorm of the rows (what those past n hold is not stored), dwconv_ln_silu's sums in its order */
 #pragma unroll
     for (int r = 0; r < DWR; ++r) {
         const float s = wave_sum(tid < D4 ? ((v[r][0] + v[r][1]) + v[r][2]) + v[r][3] : 0.0f);
@@ -648,3 +651,5 @@ extern "C" __global__ __launch_bounds__(256) void dwconv_rows(const NkDwArgs a) 
             else *(float4 *)(a.Y + (u64)(m + r) * a.D + 4 * tid) = o;
         }
 }
+extern "C" __global__ __launch_bounds__(256) void dwconv_rows(const NkDwArgs a) { dwconv_rows_impl<NK_DW_ROWS>(a); }
+extern "C" __global__ __launch_bounds__(256) void dwconv_rows_few(const NkDwArgs a) { dwconv_rows_impl<NK_DW_ROWS_FEW>(a); }

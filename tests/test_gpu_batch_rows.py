@@ -3,10 +3,10 @@
 Attention of whole chunks: windows around the 16-key tiles up to the 80-row limit, one key, fresh
 streams.  Tolerance: f32 products and sums in another order than the oracle's, 1e-5 of the largest.
 
-Depthwise conv + LN + SiLU of table rows: from 1200 rows on a workgroup takes seven table rows, with
-shared input rows where they lie on consecutive cache rows, so every row has to come out with the same
-bits however the table is cut into chunks, ordered or started; the reference is the same row in a
-table whose neighbours are elsewhere.
+Depthwise conv + LN + SiLU of table rows: from 1200 rows on a workgroup takes two table rows, from 3000
+on seven, with shared input rows where they lie on consecutive cache rows, so every row has to come out
+with the same bits however the table is cut into chunks, ordered or started; the references are the
+same row in a table whose neighbours are elsewhere and in tables of one row per workgroup.
 """
 import numpy as np
 import pytest
@@ -50,9 +50,10 @@ def test_attention_chunk_edges(gpu, spec):
     assert np.array_equal(dOs.read((m, 2 * D), np.uint16), split_rows(out))
 
 
+@pytest.mark.parametrize("rows", [1203, 3002])
 @pytest.mark.parametrize("D", [4, 256, 1020, 1024])
 @pytest.mark.parametrize("order", ["chunks", "shuffled", "middle", "descending", "gaps"])
-def test_dwconv_runs(gpu, D, order):
+def test_dwconv_runs(gpu, D, order, rows):
     import nemoasr
 
     L = nemoasr.lib()
@@ -69,7 +70,7 @@ def test_dwconv_runs(gpu, D, order):
         table = table[::-1]
     elif order == "gaps":  # indices that go on while the cache rows do not, and the reverse
         table = [(r + (i > 2), i + (i > 4), c, k) for r, i, c, k in table]
-    table = (table * (1200 // len(table) + 1))[:1203]
+    table = (table * (rows // len(table) + 1))[:rows]
     M = len(table)
     din = rng.standard_normal((pos + 8, D)).astype(np.float32)
     W = (rng.standard_normal((D, 9)) / 3).astype(np.float32)
@@ -78,14 +79,18 @@ def test_dwconv_runs(gpu, D, order):
     alone = [(table[i][0], 0, 1, 0) for i in perm]
     ddin, dW, dg, db = (gpu.put(x) for x in (din, W, g, b))
     drows, dalone = gpu.put(np.asarray(table, np.int32)), gpu.put(np.asarray(alone, np.int32))
-    dY, dYs, dA = (gpu.alloc(M * D * 4) for _ in range(3))
+    dY, dYs, dA, dO = (gpu.alloc(M * D * 4) for _ in range(4))
     gpu.begin()
+    for m in range(0, M, 1100):  # one row per workgroup
+        gpu.check(L.nk_dwconv_ln_silu_rows(gpu.h, ddin.ptr, drows.at(16 * m), min(1100, M - m), dW.ptr, dg.ptr, db.ptr,
+                                           dO.at(4 * D * m), D, 9, 1e-5))
     gpu.check(L.nk_dwconv_ln_silu_rows(gpu.h, ddin.ptr, drows.ptr, M, dW.ptr, dg.ptr, db.ptr, dY.ptr, D, 9, 1e-5))
     gpu.check(L.nk_dwconv_ln_silu_rows(gpu.h, ddin.ptr, dalone.ptr, M, dW.ptr, dg.ptr, db.ptr, dA.ptr, D, 9, 1e-5))
     gpu.check(L.nk_dwconv_ln_silu_rows_split(gpu.h, ddin.ptr, drows.ptr, M, dW.ptr, dg.ptr, db.ptr, None, dYs.ptr, D, 9, 1e-5))
     gpu.end()
     y = dY.read((M, D))
     assert np.array_equal(bits(y[perm]), bits(dA.read((M, D))))
+    assert np.array_equal(bits(y), bits(dO.read((M, D))))
     assert np.array_equal(dYs.read((M, 2 * D), np.uint16), split_rows(y))
     pick = list(range(90)) + [M - 1]
     ref = np.concatenate([oracle.dwconv_ln_silu(din[table[i][0] - 8:table[i][0] + 1], W, g, b, 1) for i in pick])
