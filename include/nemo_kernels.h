@@ -94,14 +94,15 @@ int nk_gemm_argmax(gpu_t *g, const float *A, uint32_t lda, const uint16_t *W, ui
 int nk_gemm_argmax_rows(gpu_t *g, const float *A, uint32_t lda, const uint16_t *W, uint32_t ldw, const float *bias,
                         unsigned long long *keys, uint32_t keys_ld, uint32_t M, uint32_t N, uint32_t K, uint32_t V,
                         const int *mrows, uint32_t mrows_mul);
-/* K split of the many-row residual updates (accumulate, no bias, no activation): -1 (default) by
- * operand form and tile count, 0 never, 1 always where K has more than one block.  All three give the same bits.
+/* K split of the many-row residual updates (accumulate, no bias, no activation): -1 (default) with the
+ * tile, by the same estimate, 0 never, 1 always where K has more than one block.  All three give the
+ * same bits.
  * Returns the previous setting. */
 int nk_gemm_ksplit(int mode);
 /* Many-row tile: -1 (default) by an estimate of the time from the shape, else 0 128x256 (split-row A),
  * 1 64x128, 2 64x64, 3 32x64, 4 32x32, 5 64x128 with a deeper ring (split-row A), 6 64x128 with the
- * K blocks' sum in registers (split-row residual updates), 7 96x256 (split-row A) where the tile exists
- * and divides the output columns.  All give the same bits.  Returns the previous setting. */
+ * K blocks' sum in registers (split-row residual updates), 7 96x256 (split-row A), 8 128x128 (residual
+ * updates on f32 A) where the tile exists and divides the output columns.  All give the same bits.  Returns the previous setting. */
 int nk_gemm_mx_tile(int t);
 /* Few-row residual updates (5..16 rows): 1 (default) splits K over four workgroups whose partial
  * rows are added in split order by a second launch, 0 keeps K in one workgroup (more wavefronts).

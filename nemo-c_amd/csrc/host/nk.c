@@ -8,12 +8,12 @@
 #include <string.h>
 
 static int g_force = 0;
-static int g_split = -1; /* many-row residual updates: -1 K split chosen by tile count, 0 never, 1 always */
+static int g_split = -1; /* many-row residual updates: -1 K split chosen with the tile, 0 never, 1 always */
 static int g_mx_tile = -1; /* many-row tile: -1 by estimate, else an index of mx_tile where it applies */
 
 int nk_gemm_mx_tile(int t) {
     const int prev = g_mx_tile;
-    g_mx_tile = t < 0 || t > 7 ? -1 : t;
+    g_mx_tile = t < 0 || t > 8 ? -1 : t;
     return prev;
 }
 
@@ -154,21 +154,26 @@ static uint32_t recip32(uint32_t d) { return d > 1 ? (uint32_t)(((1ull << 32) + 
  * workgroups per CU); a round takes about fix + step x K steps (64 columns) microseconds, fix1 + step1
  * x K steps when no CU has more than one workgroup.  Index 0: split-row A, fitted to FF up, FF down,
  * QKV, pw1 and out at 18 to 3584 rows (graph replays, within 15%); 1: f32 A (the split costs vector
- * work per step), fitted to the subsampling's GEMMs and joint.enc at 64 to 40128 rows. */
+ * work per step), fitted to the subsampling's GEMMs and joint.enc at 64 to 40128 rows; 2: residual
+ * updates on f32 A (their block ends take registers from the K loop), fitted at 32 to 14336 rows, N 640 to
+ * 4096, K 512 to 4096: the tile picked is within 5% of the best at each of them, 0.2% on average (with
+ * the prices of index 1 up to 36%, 8% on average). */
 typedef struct {
     const char *tile;
     uint16_t bm, bn, slots, threads, glu_threads;
-    struct { float fix, step, fix1, step1; } us[2]; /* fix 0: not built for this form */
+    struct { float fix, step, fix1, step1; } us[3]; /* fix 0: not built for this form */
+    int unsplit; /* runs all K blocks of a residual update in one workgroup */
 } mx_tile_t;
 static const mx_tile_t mx_tile[] = { /* in the order of nk_gemm_mx_tile's numbers */
-    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.70f, 5.0f, 1.65f }, { 0 } } },
-    { "64x128", 64, 128, 512, 512, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f } } },
-    { "64x64", 64, 64, 512, 512, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f } } },
-    { "32x64", 32, 64, 256, 512, 512, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f } } },
-    { "32x32", 32, 32, 256, 512, 512, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f } } },
-    { "64x128d", 64, 128, 256, 768, 512, { { 3.0f, 0.58f, 2.2f, 0.57f }, { 0 } } },
-    { "64x128u", 64, 128, 512, 256, 0, { { 3.5f, 0.95f, 3.0f, 0.76f }, { 0 } } }, /* residual updates, K not split */
-    { "96x256", 96, 256, 256, 512, 512, { { 4.0f, 1.40f, 4.0f, 1.40f }, { 0 } } },
+    { "128x256", 128, 256, 256, 512, 512, { { 5.0f, 1.70f, 5.0f, 1.65f } }, 0 },
+    { "64x128", 64, 128, 512, 512, 512, { { 4.0f, 0.95f, 3.0f, 0.74f }, { 4.2f, 1.1f, 2.0f, 0.73f }, { 4.2f, 1.40f, 3.1f, 1.14f } }, 0 },
+    { "64x64", 64, 64, 512, 512, 512, { { 2.5f, 0.70f, 2.0f, 0.33f }, { 3.4f, 0.90f, 2.2f, 0.59f }, { 2.8f, 0.82f, 4.3f, 0.56f } }, 0 },
+    { "32x64", 32, 64, 256, 512, 512, { { 1.5f, 0.29f, 1.5f, 0.29f }, { 1.7f, 0.42f, 1.7f, 0.42f }, { 3.0f, 0.39f, 4.4f, 0.39f } }, 0 },
+    { "32x32", 32, 32, 256, 512, 512, { { 1.3f, 0.25f, 1.3f, 0.25f }, { 1.7f, 0.38f, 1.7f, 0.38f }, { 2.7f, 0.37f, 4.1f, 0.37f } }, 0 },
+    { "64x128d", 64, 128, 256, 768, 512, { { 3.0f, 0.58f, 2.2f, 0.57f } }, 0 },
+    { "64x128u", 64, 128, 512, 256, 0, { { 3.5f, 0.95f, 3.0f, 0.76f } }, 1 }, /* residual updates on split rows */
+    { "96x256", 96, 256, 256, 512, 512, { { 4.0f, 1.40f, 4.0f, 1.40f } }, 0 },
+    { "128x128", 128, 128, 256, 768, 0, { { 0 }, { 0 }, { 5.2f, 1.17f, 6.1f, 0.95f } }, 0 }, /* and on f32 rows */
 };
 #define MX_TILES ((int)(sizeof mx_tile / sizeof *mx_tile))
 
@@ -181,33 +186,35 @@ static uint32_t mx_tiles(const mx_tile_t *t, uint32_t M, uint32_t nout, int glu)
 /* The tile of an (M, nout, K) GEMM, NULL when none divides the output columns, and whether its kb K
  * blocks (residual updates) run as workgroups of their own (*kz = kb) or one after another (1): the
  * least estimated time, with what each partial row after the first costs the LayerNorm that folds it
- * (3584 x 1024, three more: 6.4 us).  One after another they run on the kernel that keeps their sum in
- * registers (FF down with its LayerNorm at 3584 rows: 72 us, 77 split on 128x256), elsewhere only when
- * asked to. */
+ * (3584 x 1024, three more: 6.4 us).  One after another they run on split rows on the kernel that keeps
+ * their sum in registers (FF down with its LayerNorm at 3584 rows: 72 us, 77 split on 128x256), on
+ * its other tiles only when asked to; on f32 rows on any tile. */
 static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid, uint32_t kb,
                                 uint32_t *kz) {
     const mx_tile_t *best = NULL;
+    const int form = f32 ? (resid ? 2 : 1) : 0;
     float least = 0;
     if (nout % (glu ? 32 : 64)) return NULL;
     for (int i = 0; i < MX_TILES; ++i) {
         const mx_tile_t *t = &mx_tile[i];
-        const int unsplit = !t->glu_threads;
-        const uint32_t tiles = t->us[f32].fix > 0 && (!unsplit || (resid && g_split != 1)) ? mx_tiles(t, M, nout, glu) : 0;
+        if (!(t->us[form].fix > 0) || (t->unsplit && (!resid || g_split == 1))) continue;
+        const uint32_t tiles = mx_tiles(t, M, nout, glu);
         if (!tiles) continue;
-        const uint32_t z = unsplit || g_split == 0 || (f32 && g_split < 0 && tiles >= 400) ? 1 : kb, wgs = tiles * z;
-        if (i == g_mx_tile) {
-            *kz = z;
-            return t;
+        const int one = t->unsplit || g_split == 0 || kb == 1, both = f32 && g_split < 0 && !one;
+        for (uint32_t z = one || both ? 1 : kb;; z = kb) {
+            const uint32_t wgs = tiles * z;
+            const float steps = (float)(K / z) / NK_MX_KS;
+            const float us = (wgs <= 256 ? t->us[form].fix1 + t->us[form].step1 * steps
+                                         : (float)((wgs + t->slots - 1) / t->slots) * (t->us[form].fix + t->us[form].step * steps)) +
+                             (float)(z - 1) * (float)M * (float)nout * (4 / 6.8e6f);
+            if (!best || us < least || (i == g_mx_tile && best != t)) {
+                best = t;
+                *kz = z;
+                least = us;
+            }
+            if (one || z == kb) break;
         }
-        const float steps = (float)(K / z) / NK_MX_KS;
-        const float us = (wgs <= 256 ? t->us[f32].fix1 + t->us[f32].step1 * steps
-                                     : (float)((wgs + t->slots - 1) / t->slots) * (t->us[f32].fix + t->us[f32].step * steps)) +
-                         (float)(z - 1) * (float)M * (float)nout * (4 / 6.8e6f);
-        if (!best || us < least) {
-            best = t;
-            *kz = z;
-            least = us;
-        }
+        if (i == g_mx_tile) return t;
     }
     return best;
 }

@@ -474,5 +474,10 @@ GEMM_MX_FF(64x128, 64, 128, 2, 2, 4, 2)
 GEMM_MX_FF(64x64, 64, 64, 2, 2, 4, 3)
 GEMM_MX_FF(32x64, 32, 64, 2, 2, 4, 9)
 GEMM_MX_F(32x32, 32, 32, 2, 2, 4, 12)
+/* residual updates on f32 rows: with 64x128 a wavefront's split A, its sums and the partial row it reads
+ * back at a block's end exceed the 128 registers that two workgroups per CU leave; eight computing
+ * wavefronts on 128x128, one workgroup per CU, have 170 and half the staged weights per MFMA (3584 x 2048,
+ * K 4096, with the fold: 203 -> 175 us; 1792 x 1024, K 1024: 24.2 -> 22.5) */
+GEMM_MX(gemm_mx128x128_acc, 128, 128, 4, 2, 4, 3, false, 2, false, false)
 /* joint scores -> argmax partials (keys), 64x64 tiles: two keys per row per column tile */
 GEMM_MX(gemm_mx64x64_argmax, 64, 64, 2, 2, 4, 3, false, 1, false, false)

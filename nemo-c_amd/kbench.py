@@ -266,7 +266,7 @@ def main():
     ap.add_argument("--split-rows", default="", help="many-row GEMMs on split-row activations, e.g. 448,1792,3584")
     ap.add_argument("--tiles", default="-1", help="many-row tiles to compare (nk_gemm_mx_tile: -1 policy, "
                                                   "0 128x256, 1 64x128, 2 64x64, 3 32x64, 4 32x32, 5 64x128d, "
-                                                  "6 64x128u, 7 96x256), e.g. -1,2,1")
+                                                  "6 64x128u, 7 96x256, 8 128x128), e.g. -1,2,1")
     ap.add_argument("--ksplits", default="-1", help="residual K split modes to compare (nk_gemm_ksplit), e.g. -1,0,1")
     a = ap.parse_args()
     gpu = nemoasr.Gpu()

@@ -16,7 +16,7 @@ from test_gpu_split import bits, split_rows, w_bf16
 
 pytestmark = pytest.mark.gpu
 
-TILES = [0, 1, 2, 3, 4, 5, 6, 7, -1]
+TILES = [0, 1, 2, 3, 4, 5, 6, 7, 8, -1]
 
 
 def reference(A, W, bias, act, split):
