@@ -188,19 +188,20 @@ static uint32_t mx_tiles(const mx_tile_t *t, uint32_t M, uint32_t nout, int glu)
  * least estimated time, with what each partial row after the first costs the LayerNorm that folds it
  * (3584 x 1024, three more: 6.4 us).  One after another they run on split rows on the kernel that keeps
  * their sum in registers (FF down with its LayerNorm at 3584 rows: 72 us, 77 split on 128x256), on
- * its other tiles only when asked to; on f32 rows on any tile. */
+ * its other tiles when asked to or where the scratch holds no more than one partial row per output row
+ * (one_part); on f32 rows on any tile. */
 static const mx_tile_t *mx_pick(int f32, uint32_t M, uint32_t nout, uint32_t K, int glu, int resid, uint32_t kb,
-                                uint32_t *kz) {
+                                int one_part, uint32_t *kz) {
     const mx_tile_t *best = NULL;
-    const int form = f32 ? (resid ? 2 : 1) : 0;
+    const int form = f32 ? (resid ? 2 : 1) : 0, split = one_part ? 0 : g_split;
     float least = 0;
     if (nout % (glu ? 32 : 64)) return NULL;
     for (int i = 0; i < MX_TILES; ++i) {
         const mx_tile_t *t = &mx_tile[i];
-        if (!(t->us[form].fix > 0) || (t->unsplit && (!resid || g_split == 1))) continue;
+        if (!(t->us[form].fix > 0) || (t->unsplit && (!resid || split == 1))) continue;
         const uint32_t tiles = mx_tiles(t, M, nout, glu);
         if (!tiles) continue;
-        const int one = t->unsplit || g_split == 0 || kb == 1, both = f32 && g_split < 0 && !one;
+        const int one = t->unsplit || split == 0 || kb == 1, both = f32 && split < 0 && !one;
         for (uint32_t z = one || both ? 1 : kb;; z = kb) {
             const uint32_t wgs = tiles * z;
             const float steps = (float)(K / z) / NK_MX_KS;
@@ -229,32 +230,29 @@ static int launch_mx_s(gpu_t *g, NkGemmArgs *a, uint32_t M, uint32_t nout, uint3
                        const mx_scratch_t *sc, nk_resid_t *pend) {
     const uint32_t kb = resid ? mx_kblocks(K) : 1;
     uint32_t kz = 1;
-    const mx_tile_t *t = mx_pick(!a->A2, M, nout, K, glu, resid, kb, &kz);
+    const mx_tile_t *t = mx_pick(!a->A2, M, nout, K, glu, resid, kb, 0, &kz);
     if (!t) return 1;
-    const uint32_t tiles = mx_tiles(t, M, nout, glu);
     a->kblocks = 1;
     if (resid) {
+        /* scratch that cannot hold the split's partial rows (a fixed region, a capture that cannot grow
+         * it) may hold the unsplit ones: the tile is picked again for that (same bits: the K blocks are
+         * summed in the same order either way; split rows, 1536 x 1024, K 4096: 36 us on 64x128d, 82 on the
+         * split's tile) */
+        const size_t part = (size_t)M * nout;
+        const int fixed = sc && sc->ws;
         a->kblocks = kb;
-        const size_t need = (size_t)kz * M * nout;
-        if (sc && sc->ws) {
-            /* a fixed region too small for the split may still hold the unsplit partial rows (same
-             * bits: the K blocks are summed in the same order either way) */
-            if (need > sc->ws_floats && kz > 1 && (size_t)M * nout <= sc->ws_floats) kz = 1;
-            if ((size_t)kz * M * nout > sc->ws_floats) return -2;
-            a->ws = sc->ws;
-        } else {
-            a->ws = gpu_scratch_ws(g, need);
-            if (!a->ws && kz > 1) { /* a capture that cannot grow the scratch: unsplit, same bits */
-                kz = 1;
-                a->ws = gpu_scratch_ws(g, (size_t)M * nout);
-            }
-            if (!a->ws) return bad(g, "gemm: residual-update scratch unavailable (size it before capture)");
+        a->ws = !fixed ? gpu_scratch_ws(g, kz * part) : kz * part <= sc->ws_floats ? sc->ws : NULL;
+        if (!a->ws && kz > 1) {
+            t = mx_pick(!a->A2, M, nout, K, glu, resid, kb, 1, &kz);
+            a->ws = !fixed ? gpu_scratch_ws(g, part) : part <= sc->ws_floats ? sc->ws : NULL;
         }
+        if (!a->ws && fixed) return -2;
+        if (!a->ws) return bad(g, "gemm: residual-update scratch unavailable (size it before capture)");
         pend->parts = a->ws;
         pend->nparts = kz;
         pend->alpha = a->alpha;
     }
-    const uint32_t tm = (M + t->bm - 1) / t->bm;
+    const uint32_t tiles = mx_tiles(t, M, nout, glu), tm = (M + t->bm - 1) / t->bm;
     a->splits = kz;
     /* at most 8 row tiles per group: an XCD's 64 resident workgroups then cover about 8 row tiles x 8
      * column tiles, whose A panels stay in its L2 while the weight columns stream past (at 3584

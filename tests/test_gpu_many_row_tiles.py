@@ -40,11 +40,14 @@ def reference(A, W, bias, act, split):
 @pytest.mark.parametrize("M,N,K", [(17, 256, 64), (32, 256, 128), (33, 512, 704), (64, 256, 1024), (65, 1024, 192),
                                    (97, 512, 320), (129, 512, 1024), (300, 2048, 256), (18, 256, 96), (65, 256, 32), (70, 512, 1056),
                                    (50, 256, 2048)])
-@pytest.mark.parametrize("form", ["plain", "bias_relu", "silu_split", "glu_rows", "odd_ldc", "resid"])
+@pytest.mark.parametrize("form", ["plain", "bias_relu", "silu_split", "glu_rows", "odd_ldc", "resid", "resid_unsplit"])
 def test_tiles_agree(gpu, M, N, K, form):
+    """resid_unsplit: the K blocks one after another on every tile (partial rows read back)."""
     import nemoasr
 
     L = nemoasr.lib()
+    ksplit = 0 if form == "resid_unsplit" else -1
+    form = form.removesuffix("_unsplit")
     rng = np.random.default_rng([M, N, K])
     A = rng.standard_normal((M, K)).astype(np.float32)
     W = w_bf16(rng, N, K)
@@ -63,7 +66,7 @@ def test_tiles_agree(gpu, M, N, K, form):
         got = {}
         for tile in TILES:
             dC = gpu.alloc(M * 4 * nout) if form == "silu_split" else gpu.put(C0)
-            prev = L.nk_gemm_mx_tile(tile)
+            prev, prev_split = L.nk_gemm_mx_tile(tile), L.nk_gemm_ksplit(ksplit)
             try:
                 gpu.begin()
                 gpu.check(L.nk_gemm_split(
@@ -74,6 +77,7 @@ def test_tiles_agree(gpu, M, N, K, form):
                 gpu.end()
             finally:
                 L.nk_gemm_mx_tile(prev)
+                L.nk_gemm_ksplit(prev_split)
             got[tile] = dC.read((M, 2 * nout), np.uint16) if form == "silu_split" else dC.read((rows, ldc))
             dC.free()
         for tile in TILES:
