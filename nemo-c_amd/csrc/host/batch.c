@@ -1645,7 +1645,10 @@ int nemoasr_batch_reset_stream(nemoasr_batch_t *b, int stream, char *err, size_t
     if (dec_drain(b, err, errlen)) return -1;
     stream_clear(b, stream);
     b->st[stream].n_tok = 0;
-    if (stream_zero_device(b, stream)) { snprintf(err, errlen, "batch: reset upload failed"); return -1; }
+    if (stream_zero_device(b, stream)) {
+        snprintf(err, errlen, "batch: stream reset on the GPU failed: %s", gpu_last_error(b->g));
+        return -1;
+    }
     return 0;
 }
 

@@ -72,7 +72,10 @@ decoder_t *decoder_create(model_t *m) {
         return NULL;
     }
     d->use_graphs = 1;
-    decoder_reset(d);
+    if (decoder_reset(d)) {
+        decoder_destroy(d);
+        return NULL;
+    }
     return d;
 }
 
@@ -95,7 +98,7 @@ void decoder_destroy(decoder_t *d) {
 
 /* src/decoder.c:48-53: zero LSTM state (so Wh0 . h0 is zero too), last token blank, no valid
  * prediction */
-void decoder_reset(decoder_t *d) {
+int decoder_reset(decoder_t *d) {
     NkDecState s[2];
     memset(s, 0, sizeof s);
     s[0].last_token = d->m->cfg.blank_id;
@@ -108,7 +111,8 @@ void decoder_reset(decoder_t *d) {
     a.words = 2 * sizeof(NkDecState) / sizeof(int);
     _Static_assert(sizeof s <= sizeof a.val, "loop state fits the reset arguments");
     memcpy(a.val, s, sizeof s);
-    if (a.z0 && a.z1 && a.st) nk_stream_reset(d->g, &a);
+    if (!a.z0 || !a.z1 || !a.st) return gpu_fail(d->g, "decoder: no device memory");
+    return nk_stream_reset(d->g, &a);
 }
 double decoder_last_ms(const decoder_t *d) { return d->last_ms; }
 void decoder_use_graphs(decoder_t *d, int on) {

@@ -8,7 +8,7 @@ typedef struct decoder decoder_t;
 
 decoder_t *decoder_create(model_t *m);
 void decoder_destroy(decoder_t *d);
-void decoder_reset(decoder_t *d);
+int decoder_reset(decoder_t *d); /* 0, or -1 with gpu_last_error set: the state is then undefined */
 /* Decode `frames` rows of joint_enc (device [frames][joint_hidden]); appends token ids to out.
  * Returns the count, or -1 on error. */
 int decoder_run(decoder_t *d, const float *joint_enc, int frames, int *out, int max_out, char *err, size_t errlen);

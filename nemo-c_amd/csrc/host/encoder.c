@@ -209,7 +209,7 @@ void encoder_destroy(encoder_t *e) {
 
 /* src/encoder.c:92-103: back to the state after create; the conv history rows [0, conv_left)
  * of every layer read as zeros again */
-void encoder_reset(encoder_t *e) {
+int encoder_reset(encoder_t *e) {
     e->pending_n = 0;
     e->mel_cache_n = 0;
     e->consumed = e->emitted = 0;
@@ -222,8 +222,9 @@ void encoder_reset(encoder_t *e) {
     a.stride = e->din_stride;
     a.nbuf = (uint32_t)e->m->cfg.n_layers;
     a.n = (uint32_t)(e->conv_left * e->m->cfg.d_model);
-    if (a.base) nk_stream_reset(e->g, &a);
     e->d_frames = 0;
+    if (!a.base) return gpu_fail(e->g, "encoder: no device memory");
+    return nk_stream_reset(e->g, &a);
 }
 
 int encoder_right(const encoder_t *e) { return e->right; }

@@ -15,7 +15,7 @@ typedef struct {
 
 encoder_t *encoder_create(model_t *m, int right_context);
 void encoder_destroy(encoder_t *e);
-void encoder_reset(encoder_t *e);
+int encoder_reset(encoder_t *e); /* 0, or -1 with gpu_last_error set: the state is then undefined */
 int encoder_right(const encoder_t *e);
 int encoder_chunk_frames(const encoder_t *e);
 int encoder_chunk_mel(const encoder_t *e);

@@ -162,8 +162,9 @@ static encoder_t *encoder_for(nemoasr_t *s, int right) {
  * window: at least 1.5 s and three chunks of zeros), and the session's decoder captures, without
  * running them, its graphs of every run size for that encoder's joint.enc rows.  The encoder then
  * returns to its start state; the session's decoder state is not touched (a stream in progress at
- * another latency goes on undisturbed).  Errors are not fatal. */
-static void warm_up(nemoasr_t *s, int right) {
+ * another latency goes on undisturbed).  Errors are not fatal, except that of returning the encoder to
+ * its start state (-1). */
+static int warm_up(nemoasr_t *s, int right) {
     encoder_t *e = encoder_for(s, right);
     decoder_t *d = decoder_create(s->m);
     melfe_t *fe = melfe_create();
@@ -193,7 +194,7 @@ static void warm_up(nemoasr_t *s, int right) {
     }
     melfe_destroy(fe);
     decoder_destroy(d);
-    if (e) encoder_reset(e);
+    return e ? encoder_reset(e) : 0;
 }
 
 /* Fresh front end and empty records (open and reset). */
@@ -244,10 +245,10 @@ nemoasr_t *nemoasr_open(const char *model_dir, const char *language, int latency
     s->chain = 1; /* one-row chunks run the persistent chain where the device and model allow it */
     s->dec = decoder_create(s->m);
     if (s->dec) decoder_use_graphs(s->dec, s->graphs);
-    if (s->dec) warm_up(s, right);
+    const int warm = s->dec ? warm_up(s, right) : 0;
     s->warm = 1u << right;
     s->enc = encoder_for(s, right);
-    if (!s->enc || !s->dec || begin_stream(s)) {
+    if (!s->enc || !s->dec || warm || begin_stream(s)) {
         set_err(err, errlen, "session setup on the GPU failed: %s", gpu_last_error(s->m->gpu));
         nemoasr_close(s);
         return NULL;
@@ -385,9 +386,9 @@ int nemoasr_prepare_latency(nemoasr_t *s, int latency_ms, char *err, size_t errl
     const int right = check_latency(s->m, latency_ms, err, errlen);
     if (right < 0) return -1;
     if (!(s->warm & (1u << right))) {
-        warm_up(s, right);
-        s->warm |= 1u << right;
-        if (!s->encs[latency_index(right)]) {
+        const int rc = warm_up(s, right);
+        if (!rc) s->warm |= 1u << right;
+        if (rc || !s->encs[latency_index(right)]) {
             set_err(err, errlen, "encoder setup on the GPU failed: %s", gpu_last_error(s->m->gpu));
             return -1;
         }
@@ -404,8 +405,11 @@ int nemoasr_reset(nemoasr_t *s, const char *language, int latency_ms, char *err,
         s->done = 1;
         return -1;
     }
-    encoder_reset(s->enc);
-    decoder_reset(s->dec);
+    if (encoder_reset(s->enc) || decoder_reset(s->dec)) {
+        set_err(err, errlen, "stream reset on the GPU failed: %s", gpu_last_error(s->m->gpu));
+        s->done = 1;
+        return -1;
+    }
     s->latency_ms = latency_ms;
     if (begin_stream(s)) {
         set_err(err, errlen, "out of memory");
