@@ -42,17 +42,21 @@ __device__ __forceinline__ u32 f2bf(float f) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-/* n / d for d >= 1: hardware reciprocal, one correction of the quotient by its remainder, and
- * v_div_fixup for zeros, infinities and NaN: 5 instructions for the 10 of a general IEEE division
- * (no scaling for small or huge d).  SiLU and the sigmoid have the same errors with either: at most
- * 1.8e-7 relative over |v| <= 80, 3.8e-8 in 2-norm over |v| <= 1. */
-__device__ __forceinline__ float div_ge1(float n, float d) {
-    const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+/* n / d from r = 1 / d of the hardware: one correction of the quotient by its remainder, and
+ * v_div_fixup for zeros, infinities and NaN: 5 instructions for the 10 of a general IEEE division. */
+__device__ __forceinline__ float div_by_rcp(float n, float d, float r) {
+    const float q = n * r;
     return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
 }
-/* The reference's activation forms (src/kernels.metal:6-7): a division by 1 + e^-v, IEEE expf. */
-__device__ __forceinline__ float sigmoid_f(float v) { return div_ge1(1.0f, 1.0f + expf(-v)); }
-__device__ __forceinline__ float silu_f(float v) { return div_ge1(v, 1.0f + expf(-v)); }
+/* n / d for 1 <= d <= 2^126 (the hardware reciprocal of a larger d is subnormal and comes out as 0) */
+__device__ __forceinline__ float div_ge1(float n, float d) { return div_by_rcp(n, d, __builtin_amdgcn_rcpf(d)); }
+/* The reference's activation forms (src/kernels.metal:6-7): a division by 1 + e^-v, IEEE expf.  Below
+ * v = -87.3 the divisor exceeds 2^126: the reciprocal is taken of a quarter of it.  With this division or
+ * the general one SiLU and the sigmoid have the same errors: at most 1.8e-7 relative over |v| <= 80,
+ * 3.8e-8 in 2-norm over |v| <= 1. */
+__device__ __forceinline__ float div_1pexp(float n, float d) { return div_by_rcp(n, d, 0.25f * __builtin_amdgcn_rcpf(0.25f * d)); }
+__device__ __forceinline__ float sigmoid_f(float v) { return div_1pexp(1.0f, 1.0f + expf(-v)); }
+__device__ __forceinline__ float silu_f(float v) { return div_1pexp(v, 1.0f + expf(-v)); }
 
 /* Butterfly sum over the 64 lanes of a wavefront; every lane ends with the same total. */
 __device__ __forceinline__ float wave_sum(float v) {
