@@ -71,10 +71,25 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2(NkConvArgs a) {
 /* The same, four channels per thread (C / 4 divides 256, 16-byte aligned rows): a thread computes DW2_FB
  * neighbouring outputs of one row, whose 9 input columns x 3 rows it loads at once (two new columns
  * per output instead of three, one memory round trip per thread; the taps come through LDS, where a
- * thread's 36 are nine 16-byte reads).  Positions outside X are products with zero.
+ * thread's 36 are nine 16-byte reads).  A tap outside X is added as a
+ * product with zero, which changes nothing for a finite weight; outputs with a NaN among them are
+ * computed again skipping it, as dwconv2d_s2 does.
  * 64 windows of 19 x 33 x 256: 32.1 -> 13.3 us (52 MB read and written: 10.7 at the rate of a copy),
  * 256 windows 120 -> 44 us. */
 #define DW2_FB 4
+/* output (t1, f1) of channels c .. c + 3, tap by tap; X: the window's channel c */
+__device__ __forceinline__ floatx4 dw2_skipping(const NkConvArgs &a, const float *X, u32 c, u32 t1, u32 f1) {
+    floatx4 acc = *(const floatx4 *)(a.bias + c);
+#pragma unroll 1 /* rare: few registers and instructions */
+    for (u32 k = 0; k < 9; ++k) {
+        const int ti = (int)(2 * t1 + k / 3) - 2, fi = (int)(2 * f1 + k % 3) - 2;
+        if (ti < 0 || ti >= (int)a.T || fi < 0 || fi >= (int)a.F) continue;
+        const floatx4 v = *(const floatx4 *)(X + ((u64)ti * a.F + fi) * a.C);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += a.W[(c + e) * 9 + k] * v[e];
+    }
+    return acc;
+}
 extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
     __shared__ floatx4 taps[1024 * 9 / 4];
     const u32 C4 = a.C / 4, tid = threadIdx.x, per = 256 / C4;
@@ -103,6 +118,7 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) w[k] = taps[(c / 4) * 9 + k];
     float *Y = a.Y + (u64)blockIdx.y * a.ys + ((u64)t1 * a.F1 + f0) * a.C + c;
+    float sum = 0.0f;
 #pragma unroll
     for (int f = 0; f < DW2_FB; ++f) {
         if (f0 + f >= a.F1) break;
@@ -112,7 +128,11 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] += w[(9 * e + k) / 4][(9 * e + k) % 4] * x[k / 3][2 * f + k % 3][e];
         *(floatx4 *)(Y + (u64)f * a.C) = acc;
+        sum += (acc[0] + acc[1]) + (acc[2] + acc[3]);
     }
+    if (sum != sum) /* a NaN among them, perhaps from a weight times a position outside X */
+#pragma unroll 1
+        for (u32 f = 0; f < DW2_FB && f0 + f < a.F1; ++f) *(floatx4 *)(Y + (u64)f * a.C) = dw2_skipping(a, X, c, t1, f0 + f);
 }
 
 /* conv 0 (1 -> C channels + ReLU) followed by conv 2 (depthwise, + bias) without storing conv 0's
@@ -121,19 +141,44 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
  * in LDS.  Every conv 0 value is computed exactly as conv2d_c1_s2_relu computes it (bias, then the
  * taps in (kh, kw) order, taps outside X skipped, ReLU) and every output exactly as dwconv2d_s2
  * computes it (bias, then the taps in order, positions outside conv 0's T1 x F1 skipped), so the
- * result equals the two kernels' bit for bit (finite weights: a skipped tap is added here as a
- * product with zero).
+ * result equals the two kernels' bit for bit.  A skipped tap is added here as a product with zero,
+ * which changes nothing for a finite weight; a channel with an infinite or NaN weight is computed
+ * again by a loop that skips.
  *
  * Bound by its 63 multiply-adds per output (17 us for 64 windows of 72 rows at the full vector rate), so
  * everything else is kept out of the loop: the mel rows lie in LDS with zeros around them, so no tap
  * is tested; a thread walks its columns left to right and reads the four new mel columns of each
  * output as one 16-byte broadcast per row (seven LDS reads where every column was read by itself, 49),
  * and the conv 0 column 2 f2 of output f2, which is column 2 (f2 + 1) - 2 of the next, is kept.
- * Positions outside conv 0 are masked, not branched around.  One window of 72 rows 8.4 -> 4.4 us, 64
- * windows 73 -> 30.6, 256 windows 216 -> 103. */
+ * Positions outside conv 0 are masked, not branched around.  One window of 72 rows 8.4 -> 4.2 us, 64
+ * windows 73 -> 31.4 (the test of the weights and its loop 0.12 and 0.9 of these), 256 windows of 121
+ * rows 216 -> 143. */
 #define CONV02_PAD 7 /* LDS index of mel column 0: the four new columns of output f2 start at 4 f2 + 4 */
+#define CONV02_LDW (NK_CONV02_FMAX + 16)
+/* outputs f0 .. fe - 1 of row t2, channel c, tap by tap */
+__device__ __forceinline__ void conv02_skipping(const NkConv02Args &a, const float (*xs)[CONV02_LDW], u32 c, u32 t2, u32 f0,
+                                             u32 fe, float *Y) {
+#pragma unroll 1 /* rare: few registers and instructions */
+    for (u32 f2 = f0; f2 < fe; ++f2) {
+        float acc = a.b2[c];
+#pragma unroll 1
+        for (u32 k2 = 0; k2 < 9; ++k2) {
+            const int t1 = (int)(2 * t2 + k2 / 3) - 2, f1 = (int)(2 * f2 + k2 % 3) - 2;
+            if (t1 < 0 || t1 >= (int)a.T1 || f1 < 0 || f1 >= (int)a.F1) continue;
+            float v = a.b0[c];
+#pragma unroll 1
+            for (u32 k = 0; k < 9; ++k) {
+                const int ti = 2 * t1 + (int)(k / 3) - 2, fi = 2 * f1 + (int)(k % 3) - 2;
+                if (ti < 0 || ti >= (int)a.T || fi < 0 || fi >= (int)a.F) continue;
+                v += a.W0[c * 9 + k] * xs[2 * (k2 / 3) + k / 3][fi + CONV02_PAD];
+            }
+            acc += a.W2[c * 9 + k2] * fmaxf(v, 0.0f);
+        }
+        Y[((u64)t2 * a.F2 + f2) * a.C + c] = acc;
+    }
+}
 extern "C" __global__ __launch_bounds__(256) void conv2d_c1_dw_s2(NkConv02Args a) {
-    constexpr u32 LDW = NK_CONV02_FMAX + 16;
+    constexpr u32 LDW = CONV02_LDW;
     __shared__ __attribute__((aligned(16))) float xs[7][LDW];
     const u32 nfb = (a.F2 + a.fb - 1) / a.fb;
     const u32 t2 = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * a.fb;
@@ -157,6 +202,13 @@ extern "C" __global__ __launch_bounds__(256) void conv2d_c1_dw_s2(NkConv02Args a
 #pragma unroll
         for (int k = 0; k < 9; ++k) { w0[k] = a.W0[c * 9 + k]; w2[k] = a.W2[c * 9 + k]; }
         const float bias0 = a.b0[c], bias2 = a.b2[c];
+        float odd[3] = { 0.f, 0.f, 0.f }; /* 0, or NaN with a weight that is not finite */
+#pragma unroll
+        for (int k = 0; k < 9; ++k) odd[k % 3] += w0[k] * 0.0f + w2[k] * 0.0f;
+        if (odd[0] + odd[1] + odd[2] != 0.0f) {
+            conv02_skipping(a, xs, c, t2, f0, fe, Y);
+            continue;
+        }
         /* mel columns 4 f2 - 6 .. 4 f2 of the seven rows; conv 0's column 2 f2 - 2 of output f2 */
         float xv[7][7], keep[3];
         /* conv 0 at row 2 t2 + kh2 - 2, column f1: mel row 2 kh2 + kh, columns q .. q + 2 of xv */

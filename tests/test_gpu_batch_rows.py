@@ -141,6 +141,40 @@ def test_dwconv2d_forms(gpu, T, F, C, batch):
     assert rel_err(y[-1], oracle.dwconv2d_s2(X[-1], W, b)) < 1e-6
 
 
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("nwin,batch", [(9, 1), (23, 3), (61, 2), (64, 40)])
+def test_convs_skip_taps_outside(gpu, nwin, batch, bad):
+    """A tap outside the input is skipped, not multiplied by zero: weights that are infinite or NaN leave
+    the outputs that skip them alone.  Every form against the oracle, which skips: the same values
+    are infinite and NaN, the rest within 1e-6 (sums of nine products in one order)."""
+    import nemoasr
+
+    L = nemoasr.lib()
+    F, C = 40, 64
+    rng = np.random.default_rng(nwin)
+    X = rng.standard_normal((batch, nwin, F)).astype(np.float32)
+    W0, W2 = ((rng.standard_normal((C, 9)) / 3).astype(np.float32) for _ in range(2))
+    b0, b2 = ((0.1 * rng.standard_normal(C)).astype(np.float32) for _ in range(2))
+    for k in range(9):
+        W0[k, k] = W2[10 + k, k] = bad
+        W0[20 + k, k], W2[20 + k, 8 - k] = bad, bad
+    T1, F1 = nwin // 2 + 1, F // 2 + 1
+    T2, F2 = T1 // 2 + 1, F1 // 2 + 1
+    with np.errstate(all="ignore"):
+        y0 = np.stack([oracle.conv2d_c1_s2_relu(x, W0, b0) for x in X])
+        ref = np.stack([oracle.dwconv2d_s2(y, W2, b2) for y in y0])
+    dX, dW0, db0, dW2, db2, d0 = (gpu.put(x) for x in (X, W0, b0, W2, b2, y0))
+    dY, dZ = gpu.alloc(ref.nbytes), gpu.alloc(ref.nbytes)
+    gpu.begin()
+    gpu.check(L.nk_conv2d_c1_dw_s2_b(gpu.h, dX.ptr, dW0.ptr, db0.ptr, dW2.ptr, db2.ptr, dY.ptr, nwin, F, T1, F1, T2, F2, C, batch))
+    gpu.check(L.nk_dwconv2d_s2_b(gpu.h, d0.ptr, dW2.ptr, db2.ptr, dZ.ptr, T1, F1, T2, F2, C, batch))
+    gpu.end()
+    for got in (dY.read(ref.shape), dZ.read(ref.shape)):
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)]) and np.array_equal(np.isinf(got), np.isinf(ref))
+        assert rel_err(got[np.isfinite(ref)], ref[np.isfinite(ref)]) < 1e-6
+
+
 @pytest.mark.parametrize("T,F,C,batch", [(10, 17, 256, 12), (3, 5, 1016, 33), (9, 11, 36, 141)])
 def test_flatten_forms(gpu, T, F, C, batch):
     """Through LDS (half a million elements or more) and element by element: the transpose itself."""
