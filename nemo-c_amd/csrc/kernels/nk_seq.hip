@@ -364,7 +364,7 @@ extern "C" __global__ __launch_bounds__(512) void attention_rel(const NkAttnArgs
  * row read 64 consecutive bytes: with 32 consecutive dims per lane every load touched 64 lines of
  * which the next seven loads needed the rest, more than the L1 holds.  V granule g of row r is at
  * slot g ^ (4 (r % 4) + r / 4 % 4), which makes the column reads of the P.V product (rows 4 k .. 4 k + 3)
- * conflict-free; V is its first operand, so a lane stores four consecutive dims.   Graph-replayed, 8
+ * conflict-free; V is its first operand, so a lane stores four consecutive dims.  Graph-replayed, 8
  * heads: 23 chunks of 7 rows 10.3 -> 8.6 us, 64 of 7 16.8 -> 13.4, 256 of 14 62.4 -> 53.5 (eight
  * wavefronts 69.9: every wavefront loads the query rows again). */
 #define ATC_SLD 97 /* score row stride in floats: 96 position columns + 1 */
@@ -495,10 +495,14 @@ extern "C" __global__ __launch_bounds__(256, 3) void attention_rel_chunks(const 
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const u32 d = off + 16 * (wave + 4 * t) + 4 * kq;
-            if (a.Os) store_split4(a.Os + (u64)(m0 + qi) * 2 * a.D, a.D, d, make_float4(o[t][0], o[t][1], o[t][2], o[t][3]));
+            u16 *const os = a.Os + (u64)(m0 + qi) * 2 * a.D;
+            if (a.Os && ((size_t)a.Os & 7) == 0) store_split4(os, a.D, d, make_float4(o[t][0], o[t][1], o[t][2], o[t][3]));
             else
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a.O[(u64)(m0 + qi) * a.D + d + e] = o[t][e];
+                for (int e = 0; e < 4; ++e) {
+                    if (a.Os) store_split1(os, a.D, d + e, o[t][e]);
+                    else a.O[(u64)(m0 + qi) * a.D + d + e] = o[t][e];
+                }
         }
 }
 

@@ -37,17 +37,20 @@ def test_attention_chunk_edges(gpu, spec):
         chunks += [pos, m, c, cached]
         m += c
     dkv, dP, dbu, dbv, dch = (gpu.put(x) for x in (kv, P, bu, bv, np.asarray(chunks, np.int32)))
-    dO, dOs = gpu.alloc(m * D * 4), gpu.alloc(m * D * 4)
+    dO, dOs, dOff = gpu.alloc(m * D * 4), gpu.alloc(m * D * 4), gpu.alloc(m * D * 4 + 8)
     scale = float(np.float32(1.0) / np.sqrt(np.float32(dh)))
     gpu.begin()
     gpu.check(L.nk_attention_rel_chunks(gpu.h, dkv.ptr, 3 * D, dch.ptr, len(spec), dP.ptr, dbu.ptr, dbv.ptr, dO.ptr, Lmax, H,
                                         dh, D, scale))
     gpu.check(L.nk_attention_rel_chunks_split(gpu.h, dkv.ptr, 3 * D, dch.ptr, len(spec), dP.ptr, dbu.ptr, dbv.ptr, dOs.ptr,
                                               Lmax, H, dh, D, scale))
+    gpu.check(L.nk_attention_rel_chunks_split(gpu.h, dkv.ptr, 3 * D, dch.ptr, len(spec), dP.ptr, dbu.ptr, dbv.ptr, dOff.at(2),
+                                              Lmax, H, dh, D, scale))  # rows off 8 bytes
     gpu.end()
     out = dO.read((m, D))
     assert rel_err(out, np.concatenate(refs)) < 1e-5
     assert np.array_equal(dOs.read((m, 2 * D), np.uint16), split_rows(out))
+    assert np.array_equal(dOff.read((m, 2 * D), np.uint16, 2), split_rows(out))
 
 
 @pytest.mark.parametrize("rows", [1203, 3002])
