@@ -100,8 +100,8 @@ def test_gemm_many_rows(gpu, M, N, K, act):
 
 
 # batched multi-stream shapes (64 streams x 7 rows, 256 x 14) through the many-row MFMA kernels:
-# each tile shape (128x128, 64x128, 64x64, plain and GLU), the residual updates' K split over
-# workgroups (by tile count, never, always), row counts that are not tile multiples, K of one or
+# the tiles picked there (plain and GLU), the residual updates' K split over workgroups (by the
+# estimate, never, always), row counts that are not tile multiples, K of one or
 # two steps, row maps
 @pytest.mark.parametrize("M,N,K,act,acc,bias", [
     (448, 4096, 1024, 1, 0, False), (448, 1024, 4096, 0, 1, False), (448, 3072, 1024, 0, 0, False),
@@ -615,10 +615,12 @@ def test_subsampling_convs(gpu, nwin):
 
 @pytest.mark.parametrize("nwin,batch,F,C", [(9, 1, 128, 256), (23, 3, 128, 256), (61, 2, 128, 256),
                                           (121, 40, 128, 256), (128, 9, 128, 256), (121, 12, 128, 256),
-                                          (17, 2, 80, 96)])
+                                          (17, 2, 80, 96), (72, 4, 128, 256), (121, 140, 128, 32), (72, 13, 256, 64),
+                                          (72, 5, 44, 64), (24, 3, 36, 96)])
 def test_subsampling_conv02_fused(gpu, nwin, batch, F, C):
     """conv 0 + conv 2 in one launch equals the two launches bit for bit (and the oracle), with
-    whole-row, 4-column and 1-column workgroups (the launcher picks by rows x windows)."""
+    workgroups of 1, 3, 6, 11 and 17 columns and whole rows (the launcher picks by rows x windows),
+    the last one of a row full or short."""
     import nemoasr
 
     lib = nemoasr.lib()

@@ -96,3 +96,44 @@ def test_tiles_agree(gpu, M, N, K, form):
         if form == "odd_ldc":
             assert np.array_equal(got[2][:, nout], C0[:, nout])
         dA.free()
+
+
+@pytest.mark.parametrize("form", ["plain", "glu", "resid"])
+def test_more_tiles_than_the_reciprocals_cover(gpu, form):
+    """65536 workgroups and more: the kernels divide instead of multiplying by reciprocals (exact below
+    that).  16421 rows on 32x32 (GLU: 32x64) tiles against 64x64, all of them, bit for bit."""
+    import nemoasr
+
+    L = nemoasr.lib()
+    M, N, K = 16421, 4096, 64
+    if form == "glu":
+        M *= 2
+    if form == "resid":
+        M, N, K = 16421, 2048, 1024  # two K blocks
+    rng = np.random.default_rng(len(form))
+    nout = N // 2 if form == "glu" else N
+    dA = gpu.put(split_rows(rng.standard_normal((M, K)).astype(np.float32)))
+    dW = gpu.put(w_bf16(rng, N, K))
+    tile, tiles = (3, -(-M // 32) * (nout // 32)) if form == "glu" else (4, -(-M // 32) * (nout // 32))
+    assert tiles * (2 if form == "resid" else 1) >= 65536
+    got = []
+    prev_split = L.nk_gemm_ksplit(1 if form == "resid" else -1)
+    try:
+        for t in (tile, 2):
+            dC = gpu.alloc(M * nout * 4)
+            gpu.begin()
+            gpu.check(L.nk_fill(gpu.h, dC.ptr, M * nout, 0.5))
+            prev = L.nk_gemm_mx_tile(t)
+            try:
+                gpu.check(L.nk_gemm_split(gpu.h, None, dA.ptr, 2 * K, dW.ptr, K, None, dC.ptr, None, nout, None, M, N, K,
+                                          3 if form == "glu" else 0, int(form == "resid"), 1.0))
+            finally:
+                L.nk_gemm_mx_tile(prev)
+            gpu.end()
+            got.append(dC.read((M, nout)))
+            dC.free()
+    finally:
+        L.nk_gemm_ksplit(prev_split)
+        dA.free()
+        dW.free()
+    assert np.array_equal(bits(got[0]), bits(got[1]))
