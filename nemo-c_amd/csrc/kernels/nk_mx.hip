@@ -18,11 +18,11 @@
  * instruction (four wavefronts on a CU stream 138 GB/s, eight 217, sixteen 323, measured from L2)
  * and then waits for its fragment reads.
  *   - PW = 4: four more wavefronts only load, so the computing ones never issue a DMA; 18 rows,
- *     FF up 10.6 -> 6.5 us, 448 rows, FF up 15.9 -> 13.4, FF down 13.8 -> 12.1.  All tiles but two.
+ *     FF up 10.6 -> 6.6 us, 448 rows, FF up 15.9 -> 13.8, FF down 13.8 -> 12.1.  All tiles but three.
  *   - PW = 0: 128x256 and 96x256 computed and loaded by eight wavefronts (two per SIMD, 198 VGPRs
  *     each: no room for loaders; 192x256 spills), half the staged bytes per MFMA of 64x128: the steps of
- *     128x256 take 1.5 us, 1.2 PFLOP/s issued, the rate of a large library product here; 3584
- *     rows, FF up 81.7 -> 68 us, pw1 40.4 -> 29.0 us.
+ *     128x256 take 1.7 us, 1.26 PFLOP/s issued (a large library product here: 1.13); 3584 rows, FF up
+ *     81.7 -> 69 us, pw1 40.4 -> 29.2 us.  64x128u by four, which keep two sets of sums.
  * In both, a step's fragments are in registers one 32-K substep ahead of their MFMAs, so LDS latency
  * is covered by the other substep's MFMAs; the accumulators stay in VGPRs; the weights are the
  * MFMA's first operand, so a lane holds four consecutive output columns and stores 8 or 16 bytes at
@@ -425,12 +425,12 @@ __device__ __forceinline__ void mx_impl(const NkGemmArgs &a, lds_char_t *const s
 
 /* Tiles and ring depths.  128x256 and 96x256 take a CU each; which of the two leaves fewer CUs idle
  * depends on the rows (1300 rows, FF up in one round of 224 tiles of 96x256 29.9 us, 176 of 128x256 34.9; 3584
- * rows, QKV 49.1 against 57.1, FF up 77.3 against 69.6).  64x128 and 64x64 fit two workgroups on a CU (2 x 64 KB, 2 x 72 KB of its
+ * rows, QKV 49.1 against 57.1, FF up 77.3 against 69).  64x128 and 64x64 fit two workgroups on a CU (2 x 64 KB, 2 x 72 KB of its
  * 160 KB of LDS): one's MFMAs run while the other waits at its barrier, the better choice once there
  * are more than 256 workgroups.  64x128d (four stages), 32x64 and 32x32 take a CU each, with nearly
  * all of a 1024-column K loop's loads in flight at once: for launches of up to 256 workgroups, whose
- * time is the latency of one.  At 18 rows FF up takes 6.5 us on 32x32 tiles, 7.3 on 32x64, 8.7 on
- * 64x64; at 448 rows 13.6 on 64x128d (eight computing wavefronts, which share the epilogue; with four 15.0), 14.5
+ * time is the latency of one.  At 18 rows FF up takes 6.6 us on 32x32 tiles, 7.3 on 32x64, 8.7 on
+ * 64x64; at 448 rows 13.8 on 64x128d (eight computing wavefronts, which share the epilogue; with four 15.0), 14.5
  * on 64x64, 16.8 on 64x128.  The host chooses by a cost per
  * round (mx_tile in csrc/host/nk.c).  Second launch bound: wavefronts per SIMD where two workgroups
  * fit a CU's LDS. */

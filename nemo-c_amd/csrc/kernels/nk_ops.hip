@@ -151,8 +151,8 @@ extern "C" __global__ __launch_bounds__(256) void dwconv2d_s2_v4(NkConvArgs a) {
  * output as one 16-byte broadcast per row (seven LDS reads where every column was read by itself, 49),
  * and the conv 0 column 2 f2 of output f2, which is column 2 (f2 + 1) - 2 of the next, is kept.
  * Positions outside conv 0 are masked, not branched around.  One window of 72 rows 8.4 -> 4.2 us, 64
- * windows 73 -> 31.4 (the test of the weights and its loop 0.12 and 0.9 of these), 256 windows of 121
- * rows 216 -> 143. */
+ * windows 73 -> 31.4, 256 windows 216 -> 90 (0.12, 0.9 and 1 of these for the test of the weights and its
+ * loop). */
 #define CONV02_PAD 7 /* LDS index of mel column 0: the four new columns of output f2 start at 4 f2 + 4 */
 #define CONV02_LDW (NK_CONV02_FMAX + 16)
 /* outputs f0 .. fe - 1 of row t2, channel c, tap by tap */
@@ -290,11 +290,10 @@ extern "C" __global__ __launch_bounds__(256) void mel_frames(const NkMelArgs a) 
     }
 }
 
-/* [T][F][C] -> [T][C*F] channel-major flatten: reference src/kernels.metal:456-462.
- * One thread per output element (reads gather, writes are coalesced). */
-/* one [F][C] row of a window per workgroup through LDS (F (C + 4) floats of at most NK_FLAT_LDS, C % 4
- * == 0, 16-byte aligned), so that both the reads and the writes are whole lines; a thread's own
- * elements were C apart.  LDS rows are C + 4 floats, which spreads the reads along f over the banks.
+/* [T][F][C] -> [T][C*F] channel-major flatten (reference src/kernels.metal:456-462) of many rows: one
+ * [F][C] row of a window per workgroup through LDS (F (C + 4) floats of at most NK_FLAT_LDS, C % 4 == 0,
+ * 16-byte aligned), so that both the reads and the writes are whole lines; a thread's own elements
+ * were C apart.  LDS rows are C + 4 floats, which spreads the reads along f over the banks.
  * 64 windows of 10 x 17 x 256: 9.9 -> 6.6 us, 256 windows 30.1 -> 16.2. */
 extern "C" __global__ __launch_bounds__(256) void flatten_cf_t(const NkFlatArgs a) {
     __shared__ __attribute__((aligned(16))) float s[NK_FLAT_LDS];
@@ -315,6 +314,7 @@ extern "C" __global__ __launch_bounds__(256) void flatten_cf_t(const NkFlatArgs 
     }
 }
 
+/* The same, one thread per output element (reads gather, writes are coalesced). */
 extern "C" __global__ __launch_bounds__(256) void flatten_cf(NkFlatArgs a) {
     const u64 idx = (u64)blockIdx.x * 256 + threadIdx.x;
     const u64 total = (u64)a.T * a.C * a.F;

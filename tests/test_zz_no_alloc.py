@@ -49,8 +49,8 @@ def test_noalloc_matches_gemm_split(gpu, ksplit):
 
 
 def test_noalloc_unsplit_when_split_does_not_fit(gpu):
-    """1536 x 1024 outputs with K = 4096 are split four ways by default below ~400 tiles (6M floats
-    of partial rows, more than the array); the unsplit partial rows (1.5M floats) fit, so the call
+    """1536 x 1024 outputs with K = 4096 are split four ways where the scratch allows it (6M floats of
+    partial rows, more than the array); the unsplit partial rows (1.5M floats) fit, so the call
     succeeds with the bits of nk_gemm_split."""
     rng = np.random.default_rng(1536)
     M, N, K = 1536, 1024, 4096
