@@ -153,14 +153,14 @@ static uint32_t recip32(uint32_t d) { return d > 1 ? (uint32_t)(((1ull << 32) + 
 /* The many-row kernels (kernels/nk_mx.hip).  A launch runs in rounds of `slots` workgroups (256 CUs x
  * workgroups per CU); a round takes about fix + step x K steps (64 columns) microseconds, fix1 + step1
  * x K steps when no CU has more than one workgroup.  Index 0: split-row A, fitted to FF up, FF down,
- * QKV, pw1 and out at 18 to 3584 rows (graph replays, within 15%; from there to 57344 rows, 4096 streams of
- * 14, the tile picked is within 5% of the best of 128x256, 96x256, 64x128 and 64x128u for each of them); 1: f32 A (the split costs vector
- * work per step), fitted to the subsampling's GEMMs and joint.enc at 64 to 40128 rows (wide products, N
- * 2048 and 4096, K 256 to 4352 at 448 to 14336 rows: 0.98 to 1.4 times, on average 1.11 times as fast as
- * on 128x128 tiles of 32-column steps, picked by tile count); 2: residual
- * updates on f32 A (their block ends take registers from the K loop), fitted at 32 to 14336 rows, N 640 to
- * 4096, K 512 to 4096: the tile picked is within 5% of the best at each of them, 0.2% on average (with
- * the prices of index 1 up to 36%, 8% on average). */
+ * QKV, pw1 and out at 18 to 3584 rows (graph replays, within 15%; from there to 57344 rows, 4096 streams
+ * of 14, the tile picked is within 5% of the best of 128x256, 96x256, 64x128 and 64x128u for each of
+ * them); 1: f32 A (the split costs vector work per step), fitted to the subsampling's GEMMs and joint.enc
+ * at 64 to 40128 rows (wide products, N 2048 and 4096, K 256 to 4352 at 448 to 14336 rows: 0.98 to 1.4
+ * times, on average 1.11 times as fast as on 128x128 tiles of 32-column steps, picked by tile count);
+ * 2: residual updates on f32 A (their block ends take registers from the K loop), fitted at 32 to 14336
+ * rows, N 640 to 4096, K 512 to 4096: the tile picked is within 5% of the best at each of them, 0.2% on
+ * average (with the prices of index 1 up to 36%, 8% on average). */
 typedef struct {
     const char *tile;
     uint16_t bm, bn, slots, threads, glu_threads;
